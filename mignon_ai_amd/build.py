@@ -19,7 +19,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT_DIR = os.path.join(HERE, "_build")
 LIB = os.path.join(OUT_DIR, "libmignon_hip.so")
-SOURCES = ["gemm.hip", "kernels.hip", "sample.hip", "engine.hip", "text.cpp"]
+SOURCES = ["gemm.hip", "kernels.hip", "seq.hip", "sample.hip", "engine.hip", "text.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",

@@ -279,6 +279,36 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
+// Packed K/V ring rows (kernels.hip): a group of four 24-bit mantissas, and a row's exponent.
+struct Pk3 {
+    uint32_t x, y, z;
+};
+
+// The exponent e of a row whose largest magnitude is amax (amax * 2^-e < 2^23; e >= -120 keeps 2^e a
+// normal float, rows below 2^-97 lose their low bits).
+__device__ __forceinline__ int kv_exp(float amax) {
+    int E;
+    (void)frexpf(amax, &E);
+    return max(E - 23, -120);
+}
+
+__device__ __forceinline__ uint32_t kv_mant(float v, int e) {
+    const float r = fminf(fmaxf(rintf(ldexpf(v, -e)), -8388607.0f), 8388607.0f);
+    return (uint32_t)(int)r & 0xffffffu;
+}
+
+__device__ __forceinline__ Pk3 kv_pack(float4 v, int e) {
+    const uint32_t u0 = kv_mant(v.x, e), u1 = kv_mant(v.y, e), u2 = kv_mant(v.z, e), u3 = kv_mant(v.w, e);
+    return Pk3{u0 | (u1 << 24), (u1 >> 8) | (u2 << 16), (u2 >> 16) | (u3 << 8)};
+}
+
+__device__ __forceinline__ void stg_pk3(Pk3* p, Pk3 v) {
+    __attribute__((address_space(1))) uint32_t* q = (__attribute__((address_space(1))) uint32_t*)p;
+    q[0] = v.x;
+    q[1] = v.y;
+    q[2] = v.z;
+}
+
 __host__ __device__ constexpr int round_up(int a, int b) { return (a + b - 1) / b * b; }
 
 // Grid mapping that keeps consecutive tiles on one XCD: the dispatcher places workgroup b on XCD b % 8,

@@ -31,6 +31,7 @@
 #include "model_file.hpp"
 #include "options.hpp"
 #include "sample.hpp"
+#include "seq.hpp"
 #include "text_abi.hpp"
 
 namespace mg {
@@ -104,6 +105,27 @@ struct DevBuf {
     T* as() const { return (T*)p; }
 };
 
+// Pinned host memory that kernels read and write directly: an input region and an output region.
+struct PinnedIO {
+    uint8_t* host = nullptr;
+    uint8_t* dev = nullptr;
+    size_t in_bytes = 0;
+    PinnedIO() = default;
+    PinnedIO(const PinnedIO&) = delete;
+    PinnedIO& operator=(const PinnedIO&) = delete;
+    ~PinnedIO() {
+        if (host) (void)hipHostFree(host);
+    }
+    // allocated once, for the largest call of its owner
+    void ensure(size_t in, size_t out) {
+        if (host) return;
+        in = (in + 255) / 256 * 256;
+        HIPCHECK(hipHostMalloc((void**)&host, in + out, hipHostMallocCoherent | hipHostMallocMapped));
+        HIPCHECK(hipHostGetDevicePointer((void**)&dev, host, 0));
+        in_bytes = in;
+    }
+};
+
 struct DevBlock {
     int steps = 1, dil_base = 2, init_dil = 1;
     int8_t* w1 = nullptr; float* b1 = nullptr; float s1 = 0;  // [2Hp][3Dp] value/gate rows paired by 16
@@ -126,12 +148,12 @@ struct DevBlock {
 enum KClass : int {
     K_ROW = 0, K_GEMM_LATCH, K_SCAN, K_LATCH_STEP, K_GEMM_GLU, K_GEMM_HIGHWAY, K_GEMM_QKV, K_ATTN, K_ATTN_STEP,
     K_GEMM_OUT, K_GEMM_LOGITS, K_HEAD_COMBINE, K_GEMM_PROBS, K_BITS, K_EXPORT, K_GEMM_I8, K_SAMPLE, K_QKV_ATTN,
-    K_STEP1, K_TILE_STEP, K_NCLASS
+    K_STEP1, K_TILE_STEP, K_SEQ, K_NCLASS
 };
 const char* const kClassNames[K_NCLASS] = {
     "row_norm_pack", "gemm_latch", "latch_scan", "latch_step", "gemm_glu", "gemm_highway", "gemm_qkv",
     "attention", "attention_step", "gemm_out", "gemm_logits", "head_combine", "gemm_probs", "bits",
-    "state_export", "gemm_i8", "sample", "qkv_attention", "session_step", "tile_step"};
+    "state_export", "gemm_i8", "sample", "qkv_attention", "session_step", "tile_step", "sequence_body"};
 
 struct Profile {
     bool on = false;
@@ -224,7 +246,13 @@ struct mg_model {
     // caller-owned cancellation flag polled by batched decodes (mg_model_set_cancel); set without the lock
     std::atomic<const volatile int32_t*> cancel{nullptr};
     mg::Step1Block* s1blocks = nullptr;  // device copy of the blocks for step1_kernel
+    // the body over whole sequences in one kernel (seq.hip), where it takes the model (shape.dt > 0)
+    mg::SeqShape seq_shape;
+    int8_t* seq_stream = nullptr;
+    float* seq_vec = nullptr;
+    mg::SeqBlock* seq_blocks = nullptr;
     mg::Workspace ws;
+    mg::PinnedIO call_io;  // mg_model_call's ids and logits
     mg::Workspace* wsp = nullptr;  // while set (an allocation-free call), the workspace in use instead of ws
     mg::Profile prof;
     std::mutex mu;
@@ -463,6 +491,13 @@ void build_device_model(mg_model* m, const HostModel& hm, int max_context) {
             x.qkv = db.qkv; x.sqkv = db.sqkv; x.wo = db.wo; x.so = db.so;
         }
         if (!sb.empty()) m->s1blocks = upload(m, sb);
+    }
+    m->seq_shape = mg::seq_shape(hm, m->window > 0 ? std::min(m->window, m->cap) : m->cap);
+    if (m->seq_shape.dt > 0) {
+        const SeqPack p = seq_pack(hm, m->seq_shape, latch_base_logits(D));
+        m->seq_stream = upload(m, p.stream);
+        m->seq_vec = upload(m, p.vec);
+        m->seq_blocks = upload(m, p.blocks);
     }
     if (m->nattn > 0) {
         if (m->heads <= 0 || D % m->heads) throw Error(MG_ERR_FORMAT, "model file: attention heads must divide the state size");
@@ -970,13 +1005,46 @@ void run_body(mg_model* m, const BodyCtx& c, hipStream_t s) {
     if (m->blocks.empty()) row_call(m, M, ROW_EMBED, c.ids, nullptr, 0, nullptr, nullptr, nullptr, false, s);
 }
 
+// The same body for B sequences of T tokens in one kernel (seq.hip), which leaves the head's operand in ws.nl / ws.ns:
+// the final-normalised rows of the positions `rows` names (null: all), where it takes the model and the length. Any
+// engine option that selects one of the layered kernels selects the layered body.
+SeqArgs seq_args(mg_model* m, int B, int T, const int32_t* ids) {
+    Workspace& w = ws_of(m);
+    SeqArgs a;
+    a.shape = m->seq_shape; a.B = B; a.T = T; a.D = m->D; a.V = m->V;
+    a.heads = m->nattn ? m->heads : 0; a.dh = a.heads ? m->D / a.heads : 1; a.window = m->window; a.cap = m->cap;
+    a.nblocks = (int)m->blocks.size(); a.ids = ids; a.emb = m->emb; a.emb_scale = m->emb_scale;
+    a.stream = m->seq_stream; a.vec = m->seq_vec; a.blocks = m->seq_blocks; a.final_norm = m->final_norm;
+    a.bin = w.bin.as<float>(); a.limbs = w.nl.as<int8_t>(); a.lscale = w.ns.as<float>();
+    return a;
+}
+
+bool seq_usable(mg_model* m, int T) {
+    if (option(OPT_GEMM_KERNEL) || option(OPT_ATTENTION_KERNEL) || option(OPT_SCAN_KERNEL) || option(OPT_OPERANDS)) return false;
+    SeqArgs a;
+    a.shape = m->seq_shape; a.B = 1; a.T = T;
+    return seq_fits(a);
+}
+
+void run_seq(mg_model* m, const SeqArgs& a, hipStream_t s) {
+    double ops = 0;
+    if (m->prof.on) {
+        const double M = (double)a.B * a.T, D = m->D, H = m->H;
+        ops = 2.0 * M * (m->nbs * (D * D + 6 * D * H + 2 * D * H) + m->nattn * 4 * D * D);
+    }
+    // ids in, the final rows' limb planes and scales out
+    ProfScope ps(m->prof, K_SEQ, s, (double)a.B * a.T * (8.0 + 3.0 * m->Dp), ops);
+    HIPCHECK(launch_seq(a, s));
+}
+
 // Head over M rows of ws.cur (optionally gathered through row_map): final RMSNorm, logits GEMM with
-// per-tile softmax statistics, then the per-row combination.
+// per-tile softmax statistics, then the per-row combination. packed: the normalised rows' operand is already in
+// ws.nl / ws.ns.
 void run_head(mg_model* m, int M, const int32_t* row_map, const int32_t* tgt, float* logits_out, HeadCombineArgs hc,
-              hipStream_t s) {
+              hipStream_t s, bool packed = false) {
     Workspace& w = ws_of(m);
     // headLogits (internal/quant/stream.go:232-248)
-    row_call(m, M, ROW_SRC, nullptr, nullptr, 0, row_map, m->final_norm, nullptr, true, s);
+    if (!packed) row_call(m, M, ROW_SRC, nullptr, nullptr, 0, row_map, m->final_norm, nullptr, true, s);
     GemmArgs g = lx_args(w.nl.as<int8_t>(), w.ns.as<float>(), m->headw, m->Vp, m->Dp, M, m->V, m->head_scale);
     g.bias = m->headb; g.out = logits_out; g.ldo = m->V;
     g.stats = w.stats.as<float>(); g.stats_ld = m->Vp / LX_BN;
@@ -1357,17 +1425,25 @@ int mg_forward_batch(mg_model* m, const int32_t* ids, int B, int T, float* logit
             int32_t* ids_d = w.ids.as<int32_t>();
             if (dev) HIPCHECK(hipMemcpyAsync(ids_d, ids + row0, (size_t)M * 4, hipMemcpyDeviceToDevice, s));
             else HIPCHECK(hipMemcpyAsync(ids_d, ids + row0, (size_t)M * 4, hipMemcpyHostToDevice, s));
-            hipLaunchKernelGGL(targets_kernel, dim3((M + 255) / 256), dim3(256), 0, s, M, T, ids_d, w.tgt.as<int32_t>());
-            HIPCHECK(hipGetLastError());
-            BodyCtx c;
-            c.B = Bc; c.T = T; c.ids = ids_d;
-            run_body(m, c, s);
+            const bool seq = seq_usable(m, T);
+            {
+                ProfScope ps(m->prof, K_ROW, s, (double)M * 8.0);
+                hipLaunchKernelGGL(targets_kernel, dim3((M + 255) / 256), dim3(256), 0, s, M, T, ids_d, w.tgt.as<int32_t>());
+                HIPCHECK(hipGetLastError());
+            }
+            if (seq) {
+                run_seq(m, seq_args(m, Bc, T, ids_d), s);
+            } else {
+                BodyCtx c;
+                c.B = Bc; c.T = T; c.ids = ids_d;
+                run_body(m, c, s);
+            }
             float* lg = nullptr;
             if (logits) lg = dev ? logits + row0 * V : st.out<float>((size_t)M * V);
             HeadCombineArgs hc;
             hc.lse = w.lse.as<float>();
             hc.logprob = w.logprob.as<float>();
-            run_head(m, M, nullptr, w.tgt.as<int32_t>(), lg, hc, s);
+            run_head(m, M, nullptr, w.tgt.as<int32_t>(), lg, hc, s, seq);
             if (logprob) {
                 if (dev) HIPCHECK(hipMemcpyAsync(logprob + row0, w.logprob.p, (size_t)M * 4, hipMemcpyDeviceToDevice, s));
                 else HIPCHECK(hipMemcpyAsync(logprob + row0, w.logprob.p, (size_t)M * 4, hipMemcpyDeviceToHost, s));
@@ -1452,18 +1528,22 @@ int mg_score_sequences(mg_model* m, const int32_t* tokens, const long long* offs
         int32_t* tok_d = st.in(tokens, (size_t)n_tok, s);
         long long* start_d = st.out<long long>(max_rows);
         int32_t* len_d = st.out<int32_t>(max_rows);
+        int4* rows_d = st.out<int4>(max_rows);
         std::vector<long long> h_start;
+        std::vector<int4> h_rows;
         std::vector<int32_t> h_len, h_map, h_tgt;
         std::vector<float> h_lp;
         for (size_t r0 = 0; r0 < rows.size();) {
             const int T = rows[r0].len;
             const size_t r1 = std::min(rows.size(), r0 + (size_t)(cap / T));
             const int B = (int)(r1 - r0);
-            h_start.clear(); h_len.clear(); h_map.clear(); h_tgt.clear();
+            h_start.clear(); h_len.clear(); h_map.clear(); h_tgt.clear(); h_rows.clear();
+            const bool seq = seq_usable(m, T);  // the one-kernel body computes the scored positions' rows only
             for (size_t r = r0; r < r1; r++) {
                 const Row& row = rows[r];
                 h_start.push_back(row.start);
                 h_len.push_back(row.len);
+                h_rows.push_back(make_int4(row.first, row.count, (int)h_map.size(), 0));
                 for (int k = 0; k < row.count; k++) {
                     const int pos = row.first + k;
                     h_map.push_back((int32_t)((r - r0) * T + pos));
@@ -1473,18 +1553,25 @@ int mg_score_sequences(mg_model* m, const int32_t* tokens, const long long* offs
             const int Ms = (int)h_map.size();
             HIPCHECK(hipMemcpyAsync(start_d, h_start.data(), (size_t)B * 8, hipMemcpyHostToDevice, s));
             HIPCHECK(hipMemcpyAsync(len_d, h_len.data(), (size_t)B * 4, hipMemcpyHostToDevice, s));
-            HIPCHECK(hipMemcpyAsync(w.rowmap.p, h_map.data(), (size_t)Ms * 4, hipMemcpyHostToDevice, s));
+            if (seq) HIPCHECK(hipMemcpyAsync(rows_d, h_rows.data(), (size_t)B * sizeof(int4), hipMemcpyHostToDevice, s));
+            else HIPCHECK(hipMemcpyAsync(w.rowmap.p, h_map.data(), (size_t)Ms * 4, hipMemcpyHostToDevice, s));
             HIPCHECK(hipMemcpyAsync(w.tgt.p, h_tgt.data(), (size_t)Ms * 4, hipMemcpyHostToDevice, s));
             int32_t* ids_d = w.ids.as<int32_t>();
             hipLaunchKernelGGL(gather_rows_kernel, dim3((unsigned)(((long long)B * T + 255) / 256)), dim3(256), 0, s, B, T,
                                tok_d, start_d, len_d, ids_d);
             HIPCHECK(hipGetLastError());
-            BodyCtx c;
-            c.B = B; c.T = T; c.ids = ids_d;
-            run_body(m, c, s);
+            if (seq) {
+                SeqArgs sq = seq_args(m, B, T, ids_d);
+                sq.rows = rows_d; sq.lens = len_d;
+                run_seq(m, sq, s);
+            } else {
+                BodyCtx c;
+                c.B = B; c.T = T; c.ids = ids_d;
+                run_body(m, c, s);
+            }
             HeadCombineArgs hc;
             hc.logprob = w.logprob.as<float>();
-            run_head(m, Ms, w.rowmap.as<int32_t>(), w.tgt.as<int32_t>(), nullptr, hc, s);
+            run_head(m, Ms, w.rowmap.as<int32_t>(), w.tgt.as<int32_t>(), nullptr, hc, s, seq);
             h_lp.resize(Ms);
             HIPCHECK(hipMemcpyAsync(h_lp.data(), w.logprob.p, (size_t)Ms * 4, hipMemcpyDeviceToHost, s));
             HIPCHECK(hipStreamSynchronize(s));
@@ -1505,10 +1592,31 @@ int mg_model_call(mg_model* m, const int32_t* ids, int n, double* logits) {
             ids += n - m->max_context;
             n = m->max_context;
         }
-        std::vector<float> all((size_t)n * m->V);
-        int rc = mg_forward_batch(m, ids, 1, n, all.data(), nullptr, nullptr, nullptr, 0);
-        if (rc != MG_OK) return rc;
-        for (int v = 0; v < m->V; v++) logits[v] = (double)all[(size_t)(n - 1) * m->V + v];
+        Guard gd(m);
+        hipStream_t s = m->stream;
+        ensure_ws(m, n);
+        Workspace& w = ws_of(m);
+        // the ids and the one row of logits the caller gets live in pinned memory the kernels read and write
+        m->call_io.ensure((size_t)m->max_context * 4, (size_t)m->V * 4);
+        std::memcpy(m->call_io.host, ids, (size_t)n * 4);
+        const int32_t* ids_d = (const int32_t*)m->call_io.dev;
+        float* lg = (float*)(m->call_io.dev + m->call_io.in_bytes);
+        HeadCombineArgs hc;
+        if (seq_usable(m, n)) {
+            SeqArgs sq = seq_args(m, 1, n, ids_d);
+            sq.last_only = true;
+            run_seq(m, sq, s);
+            run_head(m, 1, nullptr, nullptr, lg, hc, s, true);
+        } else {
+            BodyCtx c;
+            c.B = 1; c.T = n; c.ids = ids_d;
+            run_body(m, c, s);
+            HIPCHECK(launch_fill_i32(w.rowmap.as<int32_t>(), 1, n - 1, s));
+            run_head(m, 1, w.rowmap.as<int32_t>(), nullptr, lg, hc, s);
+        }
+        HIPCHECK(hipStreamSynchronize(s));
+        const float* h = (const float*)(m->call_io.host + m->call_io.in_bytes);
+        for (int v = 0; v < m->V; v++) logits[v] = (double)h[v];
         return m->V;
     });
 }
@@ -1604,12 +1712,23 @@ void prefill_device(mg_sessions* s, const int32_t* prompts_d, const int32_t* len
     int32_t* lens_w = w.lens.as<int32_t>();
     hipLaunchKernelGGL(window_ids_kernel, dim3(S), dim3(128), 0, st, S, max_len, s->window, Tw, prompts_d, lens_d, ids_w, lens_w);
     HIPCHECK(hipGetLastError());
-    BodyCtx c;
-    c.B = S; c.T = Tw; c.ids = ids_w; c.sess = s; c.lens = lens_w;
-    run_body(m, c, st);
-    hipLaunchKernelGGL(last_rows_kernel, dim3((S + 255) / 256), dim3(256), 0, st, S, Tw, lens_w, w.rowmap.as<int32_t>());
-    HIPCHECK(hipGetLastError());
-    run_head(m, S, w.rowmap.as<int32_t>(), nullptr, logits_d, hc, st);
+    if (seq_usable(m, Tw)) {
+        SeqArgs sq = seq_args(m, S, Tw, ids_w);
+        sq.lens = lens_w; sq.last_only = true;
+        sq.norm_ring = s->norm_ring.as<float>(); sq.g = s->g.as<float>(); sq.ring = m->ring;
+        AttnStepArgs r;
+        ring_args(s, 0, r);
+        sq.kring = r.kring; sq.vring = r.vring; sq.kpack = r.kpack; sq.vpack = r.vpack; sq.kscale = r.kscale; sq.vscale = r.vscale;
+        run_seq(m, sq, st);
+        run_head(m, S, nullptr, nullptr, logits_d, hc, st, true);
+    } else {
+        BodyCtx c;
+        c.B = S; c.T = Tw; c.ids = ids_w; c.sess = s; c.lens = lens_w;
+        run_body(m, c, st);
+        hipLaunchKernelGGL(last_rows_kernel, dim3((S + 255) / 256), dim3(256), 0, st, S, Tw, lens_w, w.rowmap.as<int32_t>());
+        HIPCHECK(hipGetLastError());
+        run_head(m, S, w.rowmap.as<int32_t>(), nullptr, logits_d, hc, st);
+    }
     HIPCHECK(launch_set_pos(S, lens_w, s->pos.as<int32_t>(), 0, st));
 }
 

@@ -1298,28 +1298,6 @@ __device__ __forceinline__ void wave_lds_sync() {
 // kernel that reads a packed ring sees the same fp32 values and the decode kernels stay bit-identical
 // to each other.
 // ------------------------------------------------------------------------------------------------
-struct Pk3 {
-    uint32_t x, y, z;
-};
-
-// The exponent e of a row whose largest magnitude is amax (amax * 2^-e < 2^23; e >= -120 keeps 2^e a
-// normal float, rows below 2^-97 lose their low bits).
-__device__ __forceinline__ int kv_exp(float amax) {
-    int E;
-    (void)frexpf(amax, &E);
-    return max(E - 23, -120);
-}
-
-__device__ __forceinline__ uint32_t kv_mant(float v, int e) {
-    const float r = fminf(fmaxf(rintf(ldexpf(v, -e)), -8388607.0f), 8388607.0f);
-    return (uint32_t)(int)r & 0xffffffu;
-}
-
-__device__ __forceinline__ Pk3 kv_pack(float4 v, int e) {
-    const uint32_t u0 = kv_mant(v.x, e), u1 = kv_mant(v.y, e), u2 = kv_mant(v.z, e), u3 = kv_mant(v.w, e);
-    return Pk3{u0 | (u1 << 24), (u1 >> 8) | (u2 << 16), (u2 >> 16) | (u3 << 8)};
-}
-
 // Global loads and stores of one group, as three dword accesses the compiler joins into one.
 __device__ __forceinline__ Pk3 ldg_pk3(const Pk3* p) {
     const __attribute__((address_space(1))) uint32_t* q = (const __attribute__((address_space(1))) uint32_t*)p;
@@ -1329,13 +1307,6 @@ __device__ __forceinline__ Pk3 ldg_pk3_nt(const Pk3* p) {
     typedef uint32_t u3 __attribute__((ext_vector_type(3)));
     const u3 v = __builtin_nontemporal_load((const __attribute__((address_space(1))) u3*)p);
     return Pk3{v.x, v.y, v.z};
-}
-
-__device__ __forceinline__ void stg_pk3(Pk3* p, Pk3 v) {
-    __attribute__((address_space(1))) uint32_t* q = (__attribute__((address_space(1))) uint32_t*)p;
-    q[0] = v.x;
-    q[1] = v.y;
-    q[2] = v.z;
 }
 
 __device__ __forceinline__ float4 kv_unpack(Pk3 w, float s) {

@@ -51,7 +51,8 @@ _CLASSES = [("gemm_c2_kernel", "gemm_i8"), ("row_kernel", "row_norm_pack"), ("sc
             ("scan_kernel", "latch_scan"),
             ("latch_step_kernel", "latch_step"), ("attention_step", "attention_step"),
             ("qkv_attention_kernel", "qkv_attention"), ("attention", "attention"), ("head_combine_kernel", "head_combine"), ("bits_kernel", "bits"),
-            ("export_", "state_export"), ("step1_kernel", "session_step"), ("tile_step_kernel", "tile_step")]
+            ("export_", "state_export"), ("step1_kernel", "session_step"), ("tile_step_kernel", "tile_step"),
+            ("seq_kernel", "sequence_body")]
 
 
 def kernel_class(name: str) -> str:

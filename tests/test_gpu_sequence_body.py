@@ -1,0 +1,123 @@
+"""The one-kernel body (csrc/seq.hip) against the oracle and the layered kernels: every compiled variant (state of one
+or two 64-channel groups, hidden sizes of one to four, with and without attention), sequences at the edges of the
+16-token tiles and of the eight tiles of a workgroup, several sequences per workgroup, rows the head does not read,
+and the session state it exports in both ring formats."""
+import numpy as np
+import pytest
+
+from helpers import assert_close, model_bytes, oracle_model, rel_err, tiny_spec, uniform_model_bytes
+from mignon_ai_amd import Model, engine_option, synth
+from mignon_ai_amd.evaluate import score_sequences
+
+pytestmark = pytest.mark.gpu
+
+# D, H, heads, window, blocks: one entry per compiled variant, among them head widths of no whole groups of four or
+# below 16, several rule steps with dilations up to 32, a block without steps, windows of one key and of a whole tile
+SHAPES = [
+    (32, 64, 0, 0, [(2, 2, 1)]),
+    (64, 100, 0, 0, [(3, 3, 2), (1, 2, 1)]),
+    (100, 128, 0, 0, [(1, 2, 1)] * 3),
+    (128, 180, 0, 0, [(1, 2, 32)]),
+    (72, 256, 0, 0, [(2, 2, 1), (1, 2, 16)]),
+    (48, 60, 2, 64, [(1, 2, 1)] * 2),
+    (60, 128, 2, 7, [(0, 2, 1), (2, 2, 1)]),
+    (96, 128, 4, 64, [(1, 2, 1)] * 2),
+    (100, 160, 4, 1, [(1, 2, 1)] * 2),
+    (128, 256, 4, 17, [(2, 2, 1), (0, 2, 1), (1, 2, 2)]),
+]
+
+
+@pytest.fixture(autouse=True)
+def restore():
+    prev = {k: engine_option(k) for k in ("gemm", "scan", "attention", "operands", "kv_rings")}
+    yield
+    for k, v in prev.items():
+        engine_option(k, v)
+
+
+def _build(shape, seed=5):
+    D, H, heads, window, blocks = shape
+    spec = tiny_spec(blocks, V=131, D=D, H=H, heads=heads, window=window, context=128, tied=False)
+    return uniform_model_bytes(spec, seed=seed, scale=0.3)
+
+
+def _classes(m, fn):
+    m.profile(True)
+    out = fn()
+    prof = m.profile_read()
+    m.profile(False)
+    return out, prof
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_forward_lengths(shape):
+    data = _build(shape)
+    m, om = Model(data), oracle_model(data)
+    for B, T in [(1, 1), (9, 15), (17, 16), (5, 17), (3, 63), (5, 64), (3, 65), (2, 127), (3, 128)]:
+        ids = synth.token_ids(71, f"seq{shape}{T}", (B, T), 131)
+        ids[0, 0] = -3  # out of range: token 0
+        got, prof = _classes(m, lambda: m.forward_batch(ids, logits=True, logprob=True, bits=True))
+        assert "sequence_body" in prof and "gemm_glu" not in prof, (T, prof)
+        assert_close(got["logits"], om.forward_all(ids), what=f"{shape} T={T}")
+        engine_option("operands", "limbs")  # the layered body
+        want = Model(data).forward_batch(ids, logits=True, logprob=True, bits=True)
+        engine_option("operands", "auto")
+        for k in ("logits", "bits"):
+            assert_close(got[k], want[k], rtol=2e-5, what=f"{shape} T={T} {k} vs layered")
+    # longer sequences and any option that names a layered kernel take the layered body
+    ids = synth.token_ids(72, f"seq{shape}", (2, 129), 131)
+    got, prof = _classes(m, lambda: m.forward_batch(ids)["logits"])
+    assert "sequence_body" not in prof
+    assert_close(got, om.forward_all(ids), what=f"{shape} T=129")
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_call_and_score(shape):
+    """Rows the head does not read: the last position only, and windows scored at one or at all positions."""
+    data = _build(shape)
+    m, om = Model(data), oracle_model(data)
+    ids = synth.token_ids(73, f"call{shape}", (150,), 131)
+    for n in (1, 2, 16, 17, 64, 65, 80, 113, 128, 150):
+        assert_close(m.call(ids[:n]), om.call(ids[max(0, n - 128):n]), what=f"{shape} call {n}")
+    docs = [synth.token_ids(74, f"doc{n}", (n,), 131) for n in (2, 17, 40, 129, 140)]
+    for ctx in (128, 20):
+        for d, lp in zip(docs, score_sequences(m, docs, ctx)):
+            for t in range(1, len(d), 7):
+                lg = om.call(d[max(0, t - ctx):t]).astype(np.float64)
+                want = lg[d[t]] - lg.max() - np.log(np.exp(lg - lg.max()).sum())
+                assert abs(lp[t - 1] - want) <= 1e-4 * max(1.0, abs(want)), (shape, ctx, len(d), t)
+
+
+@pytest.mark.parametrize("rings", ["fp32", "packed"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_prefill_exports_the_state(shape, rings):
+    """Prefill of unequal lengths, then steps that read every part of the exported state, rings wrapping."""
+    data = _build(shape)
+    engine_option("kv_rings", rings)
+    m, om = Model(data), oracle_model(data)
+    S, T = 19, 100
+    prompts = synth.token_ids(75, f"pre{shape}", (S, T), 131)
+    lens = np.array([1, 2, 15, 16, 17, 31, 33, 48, 63, 64, 65, 66, 79, 80, 81, 96, 97, 99, 100], np.int32)
+    steps = synth.token_ids(76, f"pst{shape}", (6, S), 131)
+    s = m.sessions(S, 128)
+    (lg, am, _), prof = _classes(m, lambda: s.prefill(prompts, lens))
+    assert "sequence_body" in prof
+    out = [lg] + [s.step(steps[k])[0] for k in range(len(steps))]
+    for i in range(S):
+        for k in range(len(out)):
+            seq = np.concatenate([prompts[i, :lens[i]], steps[:k, i]])
+            assert_close(out[k][i], om.call(seq), what=f"{shape} {rings} session {i} step {k}")
+
+
+def test_forward_many_sequences():
+    """More workgroups than compute units, the benchmark's D128 model: both ends against the oracle, and against the
+    layered body everywhere."""
+    data = model_bytes("c3")
+    ids = synth.token_ids(77, "seq:c3", (600, 100), 2048)
+    got = Model(data).forward_batch(ids, logits=False, logprob=True)["logprob"]
+    engine_option("operands", "limbs")
+    want = Model(data).forward_batch(ids, logits=False, logprob=True)["logprob"]
+    engine_option("operands", "auto")
+    assert rel_err(got[:, :-1], want[:, :-1]).max() < 2e-5
+    sub = [0, 599]
+    assert_close(Model(data).forward_batch(ids[sub])["logits"], oracle_model(data).forward_all(ids[sub]), what="c3")
