@@ -361,22 +361,16 @@ __device__ __forceinline__ void lx_epilogue(const GemmArgs& g, const v4i (&acc)[
         float y[8][4];
 #pragma unroll
         for (int ti = 0; ti < 8; ti++) {
+            const int n = nb + ti * 16;
             const float4 b = *(const float4*)(bias_t + 4 * g4 + ti * 16);
             const float bb[4] = {b.x, b.y, b.z, b.w};
 #pragma unroll
             for (int r = 0; r < 4; r++) y[ti][r] = fmaf(limb_dot<B256, K512>(acc, ti, r), sw, bb[r]);
-        }
-        // (apart from the loop above, so that the eight tiles' conversions are scheduled together)
-        if (orow) {
-#pragma unroll
-            for (int ti = 0; ti < 8; ti++) {
-                if constexpr (STG) {
-                    stg_put(stg, lane, ti, y[ti]);
-                } else if (mok) {
-                    const int n = nb + ti * 16;
-                    const int nv = g.nvalid - n;
-                    if (nv > 0) store4(orow + n, y[ti], nv, vec);
-                }
+            if constexpr (STG) {
+                if (orow) stg_put(stg, lane, ti, y[ti]);
+            } else if (orow && mok) {
+                const int nv = g.nvalid - n;
+                if (nv > 0) store4(orow + n, y[ti], nv, vec);
             }
         }
         // the target logit of each token row: from the staged tile, one lane per row, when the logits are
@@ -388,8 +382,7 @@ __device__ __forceinline__ void lx_epilogue(const GemmArgs& g, const v4i (&acc)[
                 __builtin_amdgcn_wave_barrier();
                 const int t0 = row.tgt - n0;
                 if (lane < 16 && mok && t0 >= 0 && t0 < LX_BN) g.tlog[m] = stg[lane * STG_LD + t0];
-            } else if (__any(row.tgt >= n0 && row.tgt < n0 + LX_BN)) {
-                // (most tiles of a large vocabulary hold none of the wave's 16 targets)
+            } else {
                 const int t = row.tgt - nb;  // the target's position among this lane's channels
                 float tv = 0.0f;
 #pragma unroll
@@ -548,9 +541,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 //
 // Block b -> (XCD b % 8, slot b / 8); slot -> (channel slab slot % nt, run (slot / nt)*8 + XCD), so all
 // slabs of a run execute on one XCD and its activations are fetched from HBM into that XCD's L2 once.
-// Tiles whose A fragments a wave holds ahead of the one it multiplies (short K).
-constexpr int slab_depth(int epi, int kcf) { return kcf <= 2 && (epi == EPI_LOGITS || epi == EPI_PROBS) ? 2 : 1; }
-
 template <int EPI, int REM, bool STG, int KCF = 0>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_slab_kernel(GemmArgs g,
                                                                                                    int run_tiles,
@@ -589,57 +579,48 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const long long astep = 3 * 1024;  // one K step of one tile: three limb fragments
     const long long tstep = (long long)kc * astep;
 
+    const int8_t* ap = g.A + (long long)tile * tstep + lane * 16;
     if constexpr (KCF > 0) {
-        // Short K (kc == KCF): the whole A fragments of the tile DEPTH ahead are loaded right after this tile's MFMAs,
-        // before its outputs are stored. Loads and stores share one in-order completion counter, so a tile's MFMAs wait
-        // for the stores of the tile DEPTH + 1 before it: with DEPTH 1 a wave keeps one to two tiles of stores in
-        // flight (3.7 TB/s at the latency stores have under full load), with DEPTH 2 one more, where the second set of
-        // fragments fits in registers: the logits of 131072 rows, K 128, V 2048, 277 -> 207 us; K 64, 512000 rows of
-        // 512, 186 us. At K = 256 the second set spills (479 -> 717 us).
-        constexpr int DEPTH = slab_depth(EPI, KCF);
-        v4i a[DEPTH][KCF][3];
-        EpiRow row[DEPTH];
-        auto load = [&](v4i (&f)[KCF][3], EpiRow& r, int t) {
-            const int8_t* p = g.A + (long long)t * tstep + lane * 16;
+        // Short K (kc == KCF): the whole next tile's A fragments are loaded right after this tile's
+        // MFMAs, before its outputs are stored. Loads and stores share one in-order completion counter,
+        // so no load the MFMAs wait for is ever queued behind a tile's stores.
+        v4i a[KCF][3];
+#pragma unroll
+        for (int ks = 0; ks < KCF; ks++)
+#pragma unroll
+            for (int l = 0; l < 3; l++) a[ks][l] = *(const v4i*)(ap + ks * astep + l * 1024);
+        for (;;) {
+            const EpiRow row = epi_row<EPI>(g, tile * 16 + (lane & 15));
+            const int next = tile + 8;
+            const int8_t* np = next < t_end ? ap + 8 * tstep : ap;
+            v4i acc[3][8];
+#pragma unroll
+            for (int ks = 0; ks < KCF; ks++) {
+                v4i wf[8];
+                const int8_t* wp = wlane + ks * 8192;
+#pragma unroll
+                for (int ti = 0; ti < 8; ti++) wf[ti] = *(const v4i*)(wp + ti * 1024);
+#pragma unroll
+                for (int ti = 0; ti < 8; ti++)
+#pragma unroll
+                    for (int l = 0; l < 3; l++)
+                        acc[l][ti] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[ti], a[ks][l],
+                                                                           ks == 0 ? v4i{0, 0, 0, 0} : acc[l][ti], 0, 0, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 24, 0);
+            }
 #pragma unroll
             for (int ks = 0; ks < KCF; ks++)
 #pragma unroll
-                for (int l = 0; l < 3; l++) f[ks][l] = *(const v4i*)(p + ks * astep + l * 1024);
-            if constexpr (DEPTH > 1) r = epi_row<EPI>(g, t * 16 + (lane & 15));
-        };
-        // (a tile past the run's end loads the last one again: harmless, in bounds)
-#pragma unroll
-        for (int i = 0; i < DEPTH; i++) load(a[i], row[i], min(tile + 8 * i, t_end - 1));
-        for (;;) {
-#pragma unroll
-            for (int i = 0; i < DEPTH; i++) {
-                if constexpr (DEPTH == 1) row[0] = epi_row<EPI>(g, tile * 16 + (lane & 15));
-                v4i acc[3][8];
-#pragma unroll
-                for (int ks = 0; ks < KCF; ks++) {
-                    v4i wf[8];
-                    const int8_t* wp = wlane + ks * 8192;
-#pragma unroll
-                    for (int ti = 0; ti < 8; ti++) wf[ti] = *(const v4i*)(wp + ti * 1024);
-#pragma unroll
-                    for (int ti = 0; ti < 8; ti++)
-#pragma unroll
-                        for (int l = 0; l < 3; l++)
-                            acc[l][ti] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[ti], a[i][ks][l],
-                                                                               ks == 0 ? v4i{0, 0, 0, 0} : acc[l][ti], 0, 0, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x008, 24, 0);
-                }
-                const EpiRow r = row[i];
-                load(a[i], row[i], min(tile + 8 * DEPTH, t_end - 1));
-                lx_epilogue<EPI, STG, false, EPI == EPI_LOGITS || EPI == EPI_PROBS>(g, acc, tile * 16, n0, n_tile, lane,
-                                                                                    r, bias_s, stg);  // K <= 384
-                tile += 8;
-                if (tile >= t_end) return;
-            }
+                for (int l = 0; l < 3; l++) a[ks][l] = *(const v4i*)(np + ks * astep + l * 1024);
+            lx_epilogue<EPI, STG, false, EPI == EPI_LOGITS || EPI == EPI_PROBS>(g, acc, tile * 16, n0, n_tile, lane,
+                                                                                row, bias_s, stg);  // K <= 384
+            if (next >= t_end) break;
+            tile = next;
+            ap = np;
         }
+        return;
     }
-    const int8_t* ap = g.A + (long long)tile * tstep + lane * 16;
     v4i a0[3], a1[3], a2[3];
 #pragma unroll
     for (int l = 0; l < 3; l++) a0[l] = *(const v4i*)(ap + l * 1024);
@@ -1118,8 +1099,9 @@ hipError_t slab_launch(const GemmArgs& a, int grid, int lds, int run_tiles, int 
     return hipGetLastError();
 }
 
-// whole-tile prefetch for kc in {2, 4, 6}, for the head also 1; 0 when the pipelined loop is used
 constexpr bool is_head(int epi) { return epi == EPI_LOGITS || epi == EPI_PROBS; }
+
+// whole-tile prefetch for kc in {2, 4, 6}, for the head also 1; 0 when the pipelined loop is used
 template <int EPI, bool STG>
 hipError_t slab_launch_full(int kc, const GemmArgs& a, int grid, int lds, int run_tiles, int n_runs, hipStream_t stream) {
     if constexpr (is_head(EPI))
@@ -1175,8 +1157,8 @@ template <int EPI>
 hipError_t launch_any_t(const GemmArgs& a, hipStream_t stream) {
     // automatic: the weight-stationary kernel whenever its slab fits in LDS and the batch is large
     const int mode = option(OPT_GEMM_KERNEL);
-    // (one K step: only the head, whose outputs are what counts there: 512000 rows of 512 logits at K = 64 take 356 us
-    // streaming)
+    // (one K step, K = 64: only the head, whose outputs are the traffic there. Streaming them costs 356 us for 512000 rows
+    // of 512 logits, this kernel's whole row segments 186 us)
     const bool fits = (a.Kp >= 128 || is_head(EPI)) && (long long)(a.Kp / 64) * 8192 + LX_BN * 4 <= slab_lds_limit();
     const bool many = a.M >= kSlabMinRows || (a.M >= kSlabMinRowsWideK && a.Kp >= 256);
     if (fits && (mode == GEMM_SLAB || (mode == GEMM_AUTO && many))) return launch_slab_t<EPI>(a, stream);

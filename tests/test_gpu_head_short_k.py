@@ -1,4 +1,4 @@
-"""The weight-stationary head GEMM with several tiles of activations in flight (K of one or two steps of 64): row counts
+"""The weight-stationary head GEMM over one or two K steps of 64 (whole tiles of activations in flight): row counts
 at the edges of a 16-row tile, of a workgroup's eight tiles and of its run, vocabularies with partial channel tiles and
 unaligned rows, bit-identical to the streaming kernel (the same exact digit sums, the same epilogue)."""
 import numpy as np
