@@ -2301,34 +2301,17 @@ int mg_gemm_i8(const int8_t* A, int M, int K, const int8_t* W, int N, const floa
         if (M == 0) return MG_OK;
         hipStream_t st = (hipStream_t)stream;
         const bool dev = flags & MG_PTR_DEVICE;
-        const int Kp = round_up(K, GEMM_BK), Np = round_up(N, GEMM_BN);
+        // the operands as the caller has them, whatever K, N and their alignment (device pointers: in place, asynchronous)
         Staging sg;
-        // Operands in the kernel's padded layout when K or N is not a multiple of the tile; otherwise
-        // device operands are used in place.
-        const int8_t* a_d = A;
-        const int8_t* w_d = W;
-        if (!dev || Kp != K) {
-            int8_t* ap = sg.out<int8_t>((size_t)M * Kp);
-            if (Kp != K) HIPCHECK(hipMemsetAsync(ap, 0, (size_t)M * Kp, st));
-            HIPCHECK(hipMemcpy2DAsync(ap, Kp, A, K, K, M, dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, st));
-            a_d = ap;
-        }
-        if (!dev || Kp != K || Np != N) {
-            int8_t* wp = sg.out<int8_t>((size_t)Np * Kp);
-            HIPCHECK(hipMemsetAsync(wp, 0, (size_t)Np * Kp, st));
-            HIPCHECK(hipMemcpy2DAsync(wp, Kp, W, K, K, N, dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, st));
-            w_d = wp;
-        }
-        const float* s_d = dev ? scale : sg.in(scale, (size_t)N, st);
+        GemmArgs g;
+        g.A = dev ? A : sg.in(A, (size_t)M * K, st); g.a_row = K;
+        g.W = dev ? W : sg.in(W, (size_t)N * K, st); g.ldw = K;
+        g.wscale_n = dev ? scale : sg.in(scale, (size_t)N, st);
         float* c_d = C ? (dev ? C : sg.out<float>((size_t)M * N)) : nullptr;
         int32_t* i_d = acc ? (dev ? acc : sg.out<int32_t>((size_t)M * N)) : nullptr;
-        if (!c_d) c_d = sg.out<float>((size_t)M * N);
-        GemmArgs g;
-        g.A = a_d; g.a_row = Kp;
-        g.W = w_d; g.ldw = Kp; g.Np = Np; g.Kp = Kp; g.M = M; g.nvalid = N;
-        g.wscale_n = s_d; g.out = c_d; g.ldo = N; g.out_i32 = i_d;
+        g.Np = N; g.Kp = K; g.M = M; g.nvalid = N;
+        g.out = c_d; g.ldo = N; g.out_i32 = i_d;
         HIPCHECK(launch_gemm_c2(g, st));
-        if (dev && !sg.bufs.empty()) HIPCHECK(hipStreamSynchronize(st));  // padded copies die on return
         if (!dev) {
             if (C) HIPCHECK(hipMemcpyAsync(C, c_d, (size_t)M * N * 4, hipMemcpyDeviceToHost, st));
             if (acc) HIPCHECK(hipMemcpyAsync(acc, i_d, (size_t)M * N * 4, hipMemcpyDeviceToHost, st));

@@ -958,11 +958,57 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // ------------------------------------------------------------------------------------------------
 constexpr int LDSR = 80;  // LDS row stride in bytes (64 data + 16 pad)
 
+// One row of a row-major [rows][K] matrix of any K and base address, read in 16-byte pieces: a row past the last repeats
+// it (its products are not stored); bytes at K and past it are zero with ZERO, else whatever follows in the matrix
+// (they meet the other operand's zeros). Nothing outside the matrix is read.
+struct Row16 {
+    const int8_t* p;
+    int left;  // bytes from the row's start to the end of the matrix, at most K + 16
+    __device__ __forceinline__ Row16(const int8_t* base, int row, int rows, int K) {
+        const int r = min(row, rows - 1);
+        p = base + (long long)r * K;
+        left = (int)min((long long)(rows - r) * K, (long long)K + 16);
+    }
+    template <bool ZERO>
+    __device__ __forceinline__ v4i get(int k, int K) const {
+        v4i v = {0, 0, 0, 0};
+        if (k >= K) return v;
+        if (k + 16 <= left) {
+            __builtin_memcpy(&v, p + k, 16);
+        } else {
+            uint32_t t[4] = {0, 0, 0, 0};
+            for (int i = 0; i < 16; i++)
+                if (k + i < K) {
+                    const uint32_t x = (uint32_t)(uint8_t)p[k + i] << (8 * (i & 3));
+                    t[0] |= i < 4 ? x : 0;
+                    t[1] |= i >= 4 && i < 8 ? x : 0;
+                    t[2] |= i >= 8 && i < 12 ? x : 0;
+                    t[3] |= i >= 12 ? x : 0;
+                }
+            v = v4i{(int)t[0], (int)t[1], (int)t[2], (int)t[3]};
+        }
+        if (ZERO && k + 16 > K) {
+            const int n = K - k;  // 1 .. 15 valid bytes
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int have = n - 4 * i;
+                v[i] = have >= 4 ? v[i] : have <= 0 ? 0 : (int)((uint32_t)v[i] & ((1u << (8 * have)) - 1));
+            }
+        }
+        return v;
+    }
+};
+
+// RAGGED: K no multiple of 64, N no multiple of 128 or an operand or C not 16-byte aligned: operands through Row16
+// (row-major [M][K] and [N][K] as the caller has them), C in rows of 16-byte or 4-byte stores. It replaces padded copies
+// of both operands and the wait for them (they died with the call): 100000 x 500 x 1000 224 -> 164 us, 100000 x 512 x
+// 1001 292 -> 166, 20000 x 100 x 777 93 -> 28, 2 x 1446 x 308 37 -> 8.5.
+template <bool RAGGED>
 __global__ __launch_bounds__(256) void gemm_c2_kernel(GemmArgs g) {
     __shared__ __align__(16) int8_t Ws[2][GEMM_BN * LDSR];
     __shared__ __align__(16) int8_t As[2][GEMM_BM * LDSR];
 
-    const int nt = g.Np / GEMM_BN;
+    const int nt = (g.Np + GEMM_BN - 1) / GEMM_BN;
     const int mt = (g.M + GEMM_BM - 1) / GEMM_BM;
     const int total = nt * mt;
     const int t = xcd_tile(blockIdx.x, total);
@@ -978,13 +1024,24 @@ __global__ __launch_bounds__(256) void gemm_c2_kernel(GemmArgs g) {
     const int a_m = m0 + a_row_l;
     const bool a_ok = a_m < g.M;
     const int8_t* a_base = g.A + (long long)(a_ok ? a_m : 0) * g.a_row + a_col;
+    const Row16 w_row[2] = {Row16(g.W, n0 + (tid >> 2), g.nvalid, g.Kp), Row16(g.W, n0 + 64 + (tid >> 2), g.nvalid, g.Kp)};
+    const Row16 a_rowp(g.A, a_m, g.M, g.Kp);
     auto gload = [&](int k0) {
+        if constexpr (RAGGED) {
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            int c = tid + i * 256;
-            wreg[i] = *(const v4i*)(g.W + (long long)(n0 + (c >> 2)) * g.ldw + k0 + (c & 3) * 16);
+            for (int i = 0; i < 2; i++) {
+                const int c = tid + i * 256;
+                wreg[i] = w_row[i].template get<true>(k0 + (c & 3) * 16, g.Kp);
+            }
+            areg = a_rowp.template get<false>(k0 + a_col, g.Kp);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                int c = tid + i * 256;
+                wreg[i] = *(const v4i*)(g.W + (long long)(n0 + (c >> 2)) * g.ldw + k0 + (c & 3) * 16);
+            }
+            areg = a_ok ? *(const v4i*)(a_base + k0) : v4i{0, 0, 0, 0};
         }
-        areg = a_ok ? *(const v4i*)(a_base + k0) : v4i{0, 0, 0, 0};
     };
     auto sstore = [&](int buf) {
 #pragma unroll
@@ -1001,7 +1058,7 @@ __global__ __launch_bounds__(256) void gemm_c2_kernel(GemmArgs g) {
 #pragma unroll
         for (int tj = 0; tj < 2; tj++) acc[ti][tj] = v4i{0, 0, 0, 0};
 
-    const int ksteps = g.Kp / GEMM_BK;
+    const int ksteps = (g.Kp + GEMM_BK - 1) / GEMM_BK;
     gload(0);
     sstore(0);
     __syncthreads();
@@ -1022,6 +1079,52 @@ __global__ __launch_bounds__(256) void gemm_c2_kernel(GemmArgs g) {
                 acc[ti][tj] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[ti], af[tj], acc[ti][tj], 0, 0, 0);
         if (ks + 1 < ksteps) sstore(buf ^ 1);
         __syncthreads();
+    }
+
+    if constexpr (RAGGED) {
+        // C through LDS (the operand buffers are free past the loop's last barrier), half a tile at a time: 32 rows of 128,
+        // each wave storing runs of 64 consecutive channels
+        constexpr int OLD = GEMM_BN + 4;
+        float* ot = (float*)&Ws[0][0];
+        int* oi = (int*)ot;
+#pragma unroll
+        for (int tj = 0; tj < 2; tj++) {
+            auto put = [&](auto value) {
+#pragma unroll
+                for (int ti = 0; ti < 4; ti++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) oi[(wm * 16 + lrow) * OLD + wn * 64 + ti * 16 + 4 * lgrp + r] = value(ti, r);
+                __syncthreads();
+            };
+            auto get = [&](auto* out) {
+                if ((g.ldo & 3) == 0 && ((uintptr_t)out & 15) == 0) {
+                    for (int c = tid; c < 8 * GEMM_BN; c += 256) {
+                        const int row = c >> 5, n = 4 * (c & 31), m = m0 + (row >> 4) * 32 + tj * 16 + (row & 15);
+                        if (m < g.M && n0 + n < g.nvalid)  // N is a multiple of four too: whole groups
+                            __builtin_nontemporal_store(*(const f4v*)(ot + row * OLD + n), (f4v*)(out + (long long)m * g.ldo + n0 + n));
+                    }
+                } else {
+                    for (int c = tid; c < 32 * GEMM_BN; c += 256) {
+                        const int row = c >> 7, n = n0 + (c & 127), m = m0 + (row >> 4) * 32 + tj * 16 + (row & 15);
+                        if (m < g.M && n < g.nvalid)
+                            __builtin_nontemporal_store(((decltype(out))ot)[row * OLD + (c & 127)], out + (long long)m * g.ldo + n);
+                    }
+                }
+                __syncthreads();
+            };
+            if (g.out) {
+                put([&](int ti, int r) {
+                    const int n = min(n0 + wn * 64 + ti * 16 + 4 * lgrp + r, g.nvalid - 1);
+                    return __float_as_int((float)acc[ti][tj][r] * g.wscale_n[n]);
+                });
+                get(g.out);
+            }
+            if (g.out_i32) {
+                put([&](int ti, int r) { return acc[ti][tj][r]; });
+                get(g.out_i32);
+            }
+        }
+        return;
     }
 
     const int nb = n0 + wn * 64 + 4 * lgrp;
@@ -1071,13 +1174,65 @@ __global__ __launch_bounds__(256) void gemm_c2_kernel(GemmArgs g) {
             float v[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) v[r] = (float)acc[ti][tj][r] * g.wscale_n[min(n + r, g.nvalid - 1)];
-            store4(g.out + (long long)m * g.ldo + n, v, nv, (g.ldo & 3) == 0);
+            if (g.out) store4(g.out + (long long)m * g.ldo + n, v, nv, (g.ldo & 3) == 0);
             if (g.out_i32) {
                 int32_t* dst = g.out_i32 + (long long)m * g.ldo + n;
                 if (nv >= 4 && (g.ldo & 3) == 0) *(v4i*)dst = acc[ti][tj];
                 else for (int r = 0; r < 4 && r < nv; r++) dst[r] = acc[ti][tj][r];
             }
         }
+    }
+}
+
+// The plain product where its 64 x 128 tiles would leave most of the chip idle: 32 x 32 outputs per workgroup, the K steps
+// split over its four waves (operands straight from global memory in MFMA layout, any K and alignment), their exact
+// integer sums added in LDS. Bound by the operands' latency: all of a wave's loads are independent. Taken below 64 tiles:
+// 64 x 1536 x 512 (4 tiles) 11.5 -> 7.2 us, the floor of a call here; at 64 tiles (1024 x 384 x 512) the two are level,
+// at 256 (4096 x 384 x 512) this one takes 12.1 us against 7.3.
+constexpr int THIN = 32;
+constexpr int kThinTiles = 64;
+
+__global__ __launch_bounds__(256) void gemm_thin_kernel(GemmArgs g) {
+    __shared__ int part[4][THIN * (THIN + 1)];
+    const int nt = (g.nvalid + THIN - 1) / THIN;
+    const int m0 = (int)(blockIdx.x / nt) * THIN, n0 = (int)(blockIdx.x % nt) * THIN;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int lrow = lane & 15, lgrp = lane >> 4;
+    const Row16 wr[2] = {Row16(g.W, n0 + lrow, g.nvalid, g.Kp), Row16(g.W, n0 + 16 + lrow, g.nvalid, g.Kp)};
+    const Row16 ar[2] = {Row16(g.A, m0 + lrow, g.M, g.Kp), Row16(g.A, m0 + 16 + lrow, g.M, g.Kp)};
+    v4i acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[i][j] = v4i{0, 0, 0, 0};
+    const int ksteps = (g.Kp + GEMM_BK - 1) / GEMM_BK;
+#pragma unroll 2
+    for (int ks = w; ks < ksteps; ks += 4) {
+        const int k = ks * GEMM_BK + 16 * lgrp;
+        v4i wf[2], af[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++) wf[i] = wr[i].template get<true>(k, g.Kp);
+#pragma unroll
+        for (int j = 0; j < 2; j++) af[j] = ar[j].template get<false>(k, g.Kp);
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[i], af[j], acc[i][j], 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) part[w][(16 * j + lrow) * (THIN + 1) + 16 * i + 4 * lgrp + r] = acc[i][j][r];
+    __syncthreads();
+#pragma unroll
+    for (int c = tid; c < THIN * THIN; c += 256) {
+        const int row = c / THIN, col = c % THIN, m = m0 + row, n = n0 + col, o = row * (THIN + 1) + col;
+        if (m >= g.M || n >= g.nvalid) continue;
+        const int v = (part[0][o] + part[1][o]) + (part[2][o] + part[3][o]);
+        if (g.out) g.out[(long long)m * g.ldo + n] = (float)v * g.wscale_n[n];
+        if (g.out_i32) g.out_i32[(long long)m * g.ldo + n] = v;
     }
 }
 
@@ -1247,10 +1402,19 @@ hipError_t launch_gemm_fa(int epi, const GemmArgs& a, hipStream_t stream) {
 }
 
 hipError_t launch_gemm_c2(const GemmArgs& a, hipStream_t stream) {
-    if (a.Np % GEMM_BN || a.Kp % GEMM_BK || a.Kp <= 0 || a.M < 0) return hipErrorInvalidValue;
-    const int total = (a.Np / GEMM_BN) * ((a.M + GEMM_BM - 1) / GEMM_BM);
-    if (total == 0) return hipSuccess;
-    hipLaunchKernelGGL(gemm_c2_kernel, dim3(xcd_grid(total)), dim3(256), 0, stream, a);
+    if (a.Kp <= 0 || a.M < 0 || a.nvalid <= 0 || (!a.out && !a.out_i32)) return hipErrorInvalidValue;
+    if (a.M == 0) return hipSuccess;
+    const long long tiles = (long long)((a.nvalid + GEMM_BN - 1) / GEMM_BN) * ((a.M + GEMM_BM - 1) / GEMM_BM);
+    const long long thin = (long long)((a.nvalid + THIN - 1) / THIN) * ((a.M + THIN - 1) / THIN);
+    if (tiles > 0x7fffff00ll) return hipErrorInvalidValue;
+    if (tiles < kThinTiles) {
+        hipLaunchKernelGGL(gemm_thin_kernel, dim3((unsigned)thin), dim3(256), 0, stream, a);
+        return hipGetLastError();
+    }
+    const bool whole = a.Kp % GEMM_BK == 0 && a.nvalid % GEMM_BN == 0 && a.ldo % 4 == 0 && ((uintptr_t)a.out & 15) == 0 &&
+                       ((uintptr_t)a.A & 15) == 0 && ((uintptr_t)a.W & 15) == 0;
+    if (whole) hipLaunchKernelGGL(gemm_c2_kernel<false>, dim3(xcd_grid((int)tiles)), dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL(gemm_c2_kernel<true>, dim3(xcd_grid((int)tiles)), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 
