@@ -105,6 +105,8 @@ struct DevBuf {
     T* as() const { return (T*)p; }
 };
 
+constexpr int kStageSlots = 8;  // buffers a model keeps for calls with host pointers (Staging)
+
 // Pinned host memory that kernels read and write directly: an input region and an output region.
 struct PinnedIO {
     uint8_t* host = nullptr;
@@ -253,6 +255,7 @@ struct mg_model {
     mg::SeqBlock* seq_blocks = nullptr;
     mg::Workspace ws;
     mg::PinnedIO call_io;  // mg_model_call's ids and logits
+    mg::DevBuf stage[mg::kStageSlots];  // Staging's kept buffers
     mg::Workspace* wsp = nullptr;  // while set (an allocation-free call), the workspace in use instead of ws
     mg::Profile prof;
     std::mutex mu;
@@ -1066,21 +1069,43 @@ struct Guard {
     explicit Guard(mg_model* mm) : m(mm), lk(mm->mu) { HIPCHECK(hipSetDevice(mm->device)); }
 };
 
-// Host<->device staging for calls given host pointers.
+// Host<->device staging for calls given host pointers. With a model, the buffers are the model's own, one per request in
+// the order of the call, kept for its next calls (which hold the model's lock and end by waiting for the stream): an
+// allocation and its release cost more than a small call's kernels. Requests above kKeepBytes get a buffer for this call
+// only, so that a model keeps at most kKeepSlots * kKeepBytes.
+constexpr size_t kKeepBytes = 16ull << 20;
+constexpr size_t kKeepSlots = kStageSlots;
 struct Staging {
+    mg_model* m = nullptr;
+    size_t slot = 0;
     std::vector<std::unique_ptr<DevBuf>> bufs;
+    Staging() = default;
+    explicit Staging(mg_model* mm) : m(mm) {}
+    void* get(size_t bytes) {
+        bytes = std::max<size_t>(bytes, 16);
+        if (m && slot < kKeepSlots && bytes <= kKeepBytes) {
+            DevBuf& b = m->stage[slot++];
+            b.ensure(bytes);
+            return b.p;
+        }
+        bufs.emplace_back(new DevBuf());
+        bufs.back()->ensure(bytes);
+        return bufs.back()->p;
+    }
     template <class T>
     T* in(const T* host, size_t n, hipStream_t s) {
-        bufs.emplace_back(new DevBuf());
-        bufs.back()->ensure(std::max<size_t>(n * sizeof(T), 16));
-        if (n) HIPCHECK(hipMemcpyAsync(bufs.back()->p, host, n * sizeof(T), hipMemcpyHostToDevice, s));
-        return bufs.back()->as<T>();
+        T* p = (T*)get(n * sizeof(T));
+        if (n) HIPCHECK(hipMemcpyAsync(p, host, n * sizeof(T), hipMemcpyHostToDevice, s));
+        return p;
     }
     template <class T>
     T* out(size_t n) {
-        bufs.emplace_back(new DevBuf());
-        bufs.back()->ensure(std::max<size_t>(n * sizeof(T), 16));
-        return bufs.back()->as<T>();
+        return (T*)get(n * sizeof(T));
+    }
+    // the buffers of this call are free again (its work is done)
+    void reset() {
+        bufs.clear();
+        slot = 0;
     }
 };
 
@@ -1111,9 +1136,11 @@ constexpr long long kMaxChunkTokens = 1 << 21;
 // Tokens per pass for this model: kMaxChunkTokens, or fewer where the device's free memory (plus what the
 // workspace already holds, which a larger one replaces) would not hold that workspace with a quarter of
 // the free memory to spare. At least 1 (a pass that cannot be allocated then fails with MG_ERR_NOMEM).
-long long pass_tokens(mg_model* m) {
+// A call whose `need` tokens the workspace already holds takes one pass without asking the device.
+long long pass_tokens(mg_model* m, long long need) {
     Workspace& w = ws_of(m);
     if (w.cap_tokens >= kMaxChunkTokens) return kMaxChunkTokens;
+    if (need <= w.cap_tokens) return w.cap_tokens;
     if (m->wsp) return std::max(1, w.cap_tokens);  // a borrowed workspace cannot grow
     Workspace probe;
     const int sample = 1 << 16;
@@ -1414,10 +1441,10 @@ int mg_forward_batch(mg_model* m, const int32_t* ids, int B, int T, float* logit
         hipStream_t s = m->stream;
         const bool dev = flags & MG_PTR_DEVICE;
         const int V = m->V;
-        int chunk = (int)std::max<long long>(1, std::min<long long>(B, pass_tokens(m) / std::max(T, 1)));
+        int chunk = (int)std::max<long long>(1, std::min<long long>(B, pass_tokens(m, (long long)B * T) / std::max(T, 1)));
         ensure_ws(m, chunk * T);
         Workspace& w = ws_of(m);
-        Staging st;
+        Staging st(m);
         for (int b0 = 0; b0 < B; b0 += chunk) {
             const int Bc = std::min(chunk, B - b0);
             const int M = Bc * T;
@@ -1464,7 +1491,7 @@ int mg_forward_batch(mg_model* m, const int32_t* ids, int B, int T, float* logit
             if (logits && !dev) HIPCHECK(hipMemcpyAsync(logits + row0 * V, lg, (size_t)M * V * 4, hipMemcpyDeviceToHost, s));
             if (!dev) {
                 HIPCHECK(hipStreamSynchronize(s));
-                st.bufs.clear();
+                st.reset();
             }
         }
         return MG_OK;
@@ -1518,13 +1545,13 @@ int mg_score_sequences(mg_model* m, const int32_t* tokens, const long long* offs
         // every chunk holds at most `cap` row tokens (cap >= the longest row, so a chunk is never empty)
         Guard gd(m);
         const long long cap =
-            std::max<long long>(rows.empty() ? 1 : rows[0].len, std::min<long long>(pass_tokens(m), row_tokens));
+            std::max<long long>(rows.empty() ? 1 : rows[0].len, std::min<long long>(pass_tokens(m, row_tokens), row_tokens));
         const size_t max_rows = std::min<size_t>(rows.size(), (size_t)cap);
 
         hipStream_t s = m->stream;
         ensure_ws(m, (int)cap);
         Workspace& w = ws_of(m);
-        Staging st;
+        Staging st(m);
         int32_t* tok_d = st.in(tokens, (size_t)n_tok, s);
         long long* start_d = st.out<long long>(max_rows);
         int32_t* len_d = st.out<int32_t>(max_rows);
@@ -1887,7 +1914,7 @@ int mg_sessions_prefill(mg_sessions* s, const int32_t* prompts, const int32_t* l
         if (!dev)
             for (int i = 0; i < S; i++)
                 require(lens[i] >= 1 && lens[i] <= max_len, "mg_sessions_prefill: lengths must be in 1..max_len");
-        Staging sg;
+        Staging sg(m);
         const int32_t* p_d = dev ? prompts : sg.in(prompts, (size_t)S * max_len, st);
         const int32_t* l_d = dev ? lens : sg.in(lens, (size_t)S, st);
         float* lg = logits ? (dev ? logits : sg.out<float>((size_t)S * m->V)) : nullptr;
@@ -2088,7 +2115,7 @@ int mg_sessions_decode_greedy(mg_sessions* s, const int32_t* prompts, const int3
         if (!dev)
             for (int i = 0; i < S; i++)
                 require(lens[i] >= 1 && lens[i] <= max_len, "mg_sessions_decode_greedy: lengths must be in 1..max_len");
-        Staging sg;
+        Staging sg(m);
         const int32_t* p_d = dev ? prompts : sg.in(prompts, (size_t)S * max_len, st);
         const int32_t* l_d = dev ? lens : sg.in(lens, (size_t)S, st);
         int32_t* oi = dev ? out_ids : sg.out<int32_t>((size_t)S * max_tokens);
@@ -2133,7 +2160,7 @@ int mg_sessions_decode_greedy_until(mg_sessions* s, const int32_t* prompts, cons
             else HIPCHECK(launch_fill_i32(out_counts, S, 0, st));
             return MG_OK;
         }
-        Staging sg;
+        Staging sg(m);
         const int32_t* p_d = dev ? prompts : sg.in(prompts, (size_t)S * max_len, st);
         const int32_t* l_d = dev ? lens : sg.in(lens, (size_t)S, st);
         int32_t* oi = dev ? out_ids : sg.out<int32_t>((size_t)S * max_tokens);
@@ -2181,7 +2208,7 @@ int mg_sessions_decode_sample(mg_sessions* s, const int32_t* prompts, const int3
             else HIPCHECK(launch_fill_i32(out_counts, S, 0, st));
             return MG_OK;
         }
-        Staging sg;
+        Staging sg(m);
         const int32_t* p_d = dev ? prompts : sg.in(prompts, (size_t)S * max_len, st);
         const int32_t* l_d = dev ? lens : sg.in(lens, (size_t)S, st);
         const uint64_t* seed_d = dev ? seeds : sg.in(seeds, (size_t)S, st);
