@@ -15,9 +15,11 @@
 // Activations are expanded to three base-256 digits with one scale per row (scale = amax / 127, digits of
 // round(x * 127 * 65536 / amax): 0.5 / 8323072 of the row's maximum, the limb planes' own resolution).
 //
-// Weights are read once per workgroup, as a stream of units of UF fragments (1 KiB each) in the order of use: unit
-// u + 1 is in registers and unit u + 2's loads are issued when unit u's products start, two LDS slots, one barrier a
-// unit.
+// Weights are read once per workgroup, as a stream of units of UF fragments (1 KiB each) in the order of use, moved
+// straight from memory into four LDS slots: while unit u is used, units u + 1 to u + 3 are on their way, one barrier a
+// unit. A unit takes 1 to 2 thousand cycles and a load that misses the L2 about two thousand, so with only one unit
+// between a request and its use (through registers, two slots) every unit waited some 500 cycles: 1024 x 128 tokens of
+// the D128 model 756 -> 733 us, a call on 45 tokens 85.1 -> 81.8 us, scoring 60 documents 1486 -> 1432 us.
 //
 // The latch recurrence g = lambda g + (1 - lambda) n runs over the tile's tokens as a scan over the 16 lanes of a DPP
 // row (pairs (a, b) composed in four steps), then over the tiles through LDS (each tile's composed pair).
@@ -28,7 +30,7 @@
 // log-probabilities 1277 -> 704 us (of which the head takes 300); 300 x 100 tokens of D96 H160 464 -> 281 us; 64 x 128
 // of D32 H64 123 -> 43 us; the next-token call on 45 tokens of D96 H160, its head over one row instead of 45, 253 ->
 // 85 us; scoring 60 documents with the D128 model, its last block only where a scored position depends on it, 3057 ->
-// 1515 us.
+// 1515 us (all with the weights through registers).
 #include <cmath>
 #include <cstring>
 #include <type_traits>
@@ -46,6 +48,9 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 
+// Units of the weight stream in LDS: the one in use and three on their way.
+constexpr int kSlots = 4;
+
 template <int DT, int HT, int ND>
 struct Cfg {
     static constexpr int Dp = 64 * DT, Hp = 64 * HT;
@@ -55,11 +60,15 @@ struct Cfg {
     static constexpr int KS = 16 * ND + 4;   // row stride of a head's keys
     static constexpr int VS = kSeqMaxT + 4;  // row stride of a head's transposed values
     static constexpr int NV = Dp + 2 * Hp + 4 * Dp;  // vector floats in LDS: latch base, b1, b2, gamma, attention gamma
-    static constexpr int o_x = 2 * UF * 1024;
+    static constexpr int o_x = kSlots * UF * 1024;
     static constexpr int o_k = o_x + kSeqMaxT * XS * 4;
     static constexpr int o_v = o_k + (ND ? kSeqMaxT * KS * 4 : 0);
-    static constexpr int o_carry = o_v + (ND ? 16 * ND * VS * 4 : 0);
-    static constexpr int o_nmax = o_carry + 8 * Dp * 8;
+    // The tiles' composed pairs. With attention they lie on the keys: a rule step is over, and the units of its products
+    // lie between, when a head's keys are written, and the output product's units when the next block's pairs are.
+    static constexpr int o_carry = ND ? o_k : o_v;
+    static constexpr int carry = 8 * Dp * 8;
+    static_assert(ND == 0 || carry <= kSeqMaxT * KS * 4 + 16 * ND * VS * 4, "");
+    static constexpr int o_nmax = ND ? o_v + 16 * ND * VS * 4 : o_carry + carry;
     static constexpr int o_vec = o_nmax + kSeqMaxT * 4;
     static constexpr int lds = o_vec + NV * 4;
     // Waves per SIMD: four (two workgroups per CU, 128 registers) where a 64-channel state without attention leaves the
@@ -71,6 +80,22 @@ __device__ __forceinline__ void wg_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// One 16-byte load per lane from global memory straight into LDS: lane L's bytes land at LDS offset lds + 16 L. Inline
+// assembly, with the waits written out (vm_wait), because the compiler would wait for all such loads before any LDS read.
+// The LDS address goes through M0, which nothing else in this file's device code uses; the s_nop is the wait state
+// between the write of M0 and its use. No register receives anything.
+__device__ __forceinline__ void lds_load16(const void* g, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds) : "memory");
+}
+__device__ __forceinline__ uint32_t lds_offset(const void* p) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+// At most N of this wave's memory operations are outstanding (they complete in order).
+template <int N>
+__device__ __forceinline__ void vm_wait() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
 }
 
 // A value computed at this point: without it the compiler moves the last steps of each output to its use, units later,
@@ -267,28 +292,31 @@ __global__ __launch_bounds__(512)
     const bool out_act = in_rows && 16 * tile + 15 >= rows.x;
     const bool key_act = in_rows && 16 * tile + 15 >= rows.x - span + 1;
 
-    // The weight stream: unit u in LDS slot u & 1, unit u + 1 in registers when unit u begins.
+    // The weight stream: wave w moves fragments w and w + 8 of every unit, unit u to LDS slot u & 3.
     const int8_t* wp = a.stream + w * 1024 + lane * 16;
-    v4i pre0 = v4i{0, 0, 0, 0}, pre1 = v4i{0, 0, 0, 0};
-    auto fetch = [&]() {
-        if (w < C::UF) pre0 = ldg((const v4i*)wp);
-        if (C::UF > 8 && w + 8 < C::UF) pre1 = ldg((const v4i*)(wp + 8192));
+    const uint32_t slots = lds_offset(smem) + w * 1024;
+    auto request = [&](int u) {
+        const uint32_t d = slots + (u & (kSlots - 1)) * (C::UF * 1024);
+        if (C::UF >= 8 || w < C::UF) lds_load16(wp, d);
+        if (C::UF > 8 && w + 8 < C::UF) lds_load16(wp + 8192, d + 8192);
         wp += C::UF * 1024;
     };
-    auto store = [&](int sl) {
-        int8_t* d = smem + sl * C::UF * 1024 + tid * 16;
-        if (w < C::UF) *(v4i*)d = pre0;
-        if (C::UF > 8 && w + 8 < C::UF) *(v4i*)(d + 8192) = pre1;
+    // this wave's fragments of all units but the `newer` last requested have arrived
+    auto arrived = [&](auto newer) {
+        constexpr int N = decltype(newer)::value;
+        if (C::UF > 8 && w + 8 < C::UF) vm_wait<2 * N>();
+        else vm_wait<N>();
     };
     int u = 0;
-    // a unit: `begin` puts the next unit's fragments where `end` makes them readable and requests the one after it
+    // a unit: `begin` requests the unit three later into the slot that the last `end` freed, `end` makes the next unit
+    // readable
     auto begin = [&]() -> const int8_t* {
-        store((u + 1) & 1);
-        fetch();
+        request(u + kSlots - 1);
         __builtin_amdgcn_sched_barrier(0);
-        return smem + (u & 1) * C::UF * 1024 + lane * 16;
+        return smem + (u & (kSlots - 1)) * C::UF * 1024 + lane * 16;
     };
     auto end = [&]() {
+        arrived(std::integral_constant<int, kSlots - 2>{});
         wg_barrier();
         u++;
     };
@@ -316,12 +344,11 @@ __global__ __launch_bounds__(512)
 
     // out-of-range ids are token 0, as are the positions past the sequence
     int id = mine && t < a.T ? a.ids[(long long)b * a.T + t] : 0;
-    fetch();
-    store(0);
-    fetch();
+    for (int i = 0; i < kSlots - 1; i++) request(i);
     if (tid < Dp / 4) *(float4*)(smem + C::o_vec + 16 * tid) = *(const float4*)(a.vec + 4 * tid);
     vec_load(0);
     if (16 * tile >= len) {
+        arrived(std::integral_constant<int, kSlots - 2>{});
         wg_barrier();
         for (int blk = 0; blk < a.nblocks; blk++) {
             idle_units(a.blocks[blk].steps * (DT + RULE2));
@@ -331,6 +358,7 @@ __global__ __launch_bounds__(512)
                 wg_barrier();
             }
         }
+        vm_wait<0>();
         return;
     }
 
@@ -362,6 +390,7 @@ __global__ __launch_bounds__(512)
 #pragma unroll
         for (int r = 0; r < 4; r++) cur[4 * ti + r] = e[r];
     }
+    arrived(std::integral_constant<int, kSlots - 2>{});
     wg_barrier();
 
     // RMSNorm of the state rows (nn.RMSNormForwardF32): 1/rms from the mean square, then times gamma
@@ -443,6 +472,7 @@ __global__ __launch_bounds__(512)
             if (last_blk && st + 1 == steps && !(B.attn ? key_act : out_act)) {
                 idle_units(RULE2);
                 if (ND > 0 && B.attn) idle_attention();
+                vm_wait<0>();
                 return;
             }
             v4i xd[3 * DT][3];
@@ -590,6 +620,7 @@ __global__ __launch_bounds__(512)
                 const bool qo = !last_blk || out_act;
                 if (last_blk && !key_act) {  // (a last block without rule steps)
                     idle_attention();
+                    vm_wait<0>();
                     return;
                 }
                 v4i nd[DT][3];
@@ -717,6 +748,7 @@ __global__ __launch_bounds__(512)
                 ab++;
                 if (!qo) {
                     idle_units(DT);
+                    vm_wait<0>();
                     return;
                 }
                 float osw;
@@ -773,6 +805,7 @@ __global__ __launch_bounds__(512)
             wg_barrier();
         }
     }
+    vm_wait<0>();  // nothing lands in LDS after the workgroup's end
     if (!out_act) return;
 
     // the head's operand: final RMSNorm, limb planes in the GEMM's own channel order
@@ -940,7 +973,7 @@ SeqPack seq_pack(const HostModel& hm, SeqShape sh, const std::vector<float>& lat
         for (int c = 0; c < Dp; c++) p.vec.push_back(b.norm && c < D ? hb.gamma[c] : 0.0f);
         for (int c = 0; c < Dp; c++) p.vec.push_back(hb.has_attn && c < D ? hb.attn_norm[c] : 0.0f);
     }
-    p.stream.resize(p.stream.size() + (size_t)2 * UF * 1024, 0);  // the two units requested past the last one
+    p.stream.resize(p.stream.size() + (size_t)(kSlots - 1) * UF * 1024, 0);  // the units requested past the last one
     return p;
 }
 
