@@ -691,19 +691,44 @@ __global__ void targets_kernel(int M, int T, const int32_t* ids, int32_t* tgt) {
     tgt[m] = (m % T) < T - 1 ? ids[m + 1] : -1;
 }
 
-__global__ void last_rows_kernel(int B, int T, const int32_t* lens, int32_t* rowmap) {
+__global__ void last_rows_kernel(int B, int T, const int32_t* lens, const int32_t* row0, int32_t* rowmap) {
     int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < B) rowmap[b] = b * T + lens[b] - 1;
+    if (b < B) rowmap[b] = (row0 ? row0[b] : b * T) + lens[b] - 1;
+}
+
+// First rows of packed prompts (window_ids_kernel's lengths): the running sum of their whole tiles. One workgroup, a run
+// of prompts per thread.
+__global__ __launch_bounds__(1024) void pack_rows_kernel(int S, int max_len, int window, const int32_t* lens, int32_t* row0) {
+    __shared__ int32_t sums[1024];
+    const int j = threadIdx.x, n = (S + 1023) / 1024, i0 = min(j * n, S), i1 = min(i0 + n, S);
+    auto rows = [&](int i) { return packed_rows(min(min(max(lens[i], 1), max_len), window)); };
+    int own = 0;
+    for (int i = i0; i < i1; i++) own += rows(i);
+    sums[j] = own;
+    __syncthreads();
+    for (int d = 1; d < 1024; d <<= 1) {
+        const int v = j >= d ? sums[j - d] : 0;
+        __syncthreads();
+        sums[j] += v;
+        __syncthreads();
+    }
+    int at = sums[j] - own;
+    for (int i = i0; i < i1; i++) {
+        row0[i] = at;
+        at += rows(i);
+    }
 }
 
 // Prompt windowing (quantSession.Prefill keeps the last `window` tokens, internal/quant/session.go:30-39)
-// into a [S][Tw] token matrix padded with id 0; lengths are clamped to 1..max_len.
+// into a [S][Tw] token matrix padded with id 0, or with row0 into packed rows; lengths are clamped to 1..max_len.
 __global__ void window_ids_kernel(int S, int max_len, int window, int Tw, const int32_t* in, const int32_t* lens_in,
-                                  int32_t* out, int32_t* lens_out) {
+                                  const int32_t* row0, int32_t* out, int32_t* lens_out) {
     int s = blockIdx.x;
     int len = min(max(lens_in[s], 1), max_len);
     int L = min(len, window), off = len - L;
-    for (int t = threadIdx.x; t < Tw; t += blockDim.x) out[(long long)s * Tw + t] = t < L ? in[(long long)s * max_len + off + t] : 0;
+    const long long at = row0 ? row0[s] : (long long)s * Tw;
+    const int n = row0 ? packed_rows(L) : Tw;
+    for (int t = threadIdx.x; t < n; t += blockDim.x) out[at + t] = t < L ? in[(long long)s * max_len + off + t] : 0;
     if (threadIdx.x == 0) lens_out[s] = L;
 }
 
@@ -763,11 +788,14 @@ struct BodyCtx {
     mg_sessions* sess = nullptr;
     bool step = false;
     const int32_t* lens = nullptr;  // prefill export lengths (device)
+    // Packed prefill: sequence b is packed_rows(lens[b]) rows from row0[b] on, `rows` in all (ids in that order).
+    const int32_t* row0 = nullptr;
+    int rows = 0;
 };
 
 void run_body(mg_model* m, const BodyCtx& c, hipStream_t s) {
     Workspace& w = ws_of(m);
-    const int M = c.B * c.T;
+    const int M = c.row0 ? c.rows : c.B * c.T;
     const int Dp = m->Dp, Hp = m->Hp, D = m->D;
     int bs = 0, ab = 0;
     // The inter-block residual (blockIn += cur; cur = blockIn, stream.go:157-163) is done by the last GEMM
@@ -781,6 +809,7 @@ void run_body(mg_model* m, const BodyCtx& c, hipStream_t s) {
     const int sk = option(OPT_SCAN_KERNEL);
     const bool many = (long long)c.B * ((Dp / 2 + 63) / 64) >= 1024;
     auto fused_scan_at = [&](const DevBlock& blk, int st) {
+        if (c.row0) return true;  // (prefill_packs)
         return !c.step && scan_rule_fits(c.T, Dp, blk.dilation(st)) && (sk == 2 || (sk == 0 && many));
     };
     // The latch GEMM of a block whose input is in blockIn (added there by the previous block's last GEMM)
@@ -861,11 +890,11 @@ void run_body(mg_model* m, const BodyCtx& c, hipStream_t s) {
                 sa.B = c.B; sa.T = c.T; sa.D = D; sa.Dp = Dp;
                 sa.lam = w.lam.as<float>(); sa.nf = w.nf.as<float>(); sa.g = w.lam.as<float>();
                 if (c.sess) {
-                    sa.lens = c.lens;
+                    sa.lens = c.lens; sa.row0 = c.row0;
                     sa.g_out = c.sess->g.as<float>() + (size_t)bs * c.B * Dp;
                     ProfScope ps(m->prof, K_EXPORT, s);
                     HIPCHECK(launch_export_ring(c.B, c.T, Dp, m->ring, c.lens, w.nf.as<float>(),
-                                                c.sess->norm_ring.as<float>() + (size_t)bs * c.B * m->ring * Dp, s));
+                                                c.sess->norm_ring.as<float>() + (size_t)bs * c.B * m->ring * Dp, s, c.row0));
                 }
                 // rule input [n | left | g] (stream.go:180-184), limb-expanded with one scale per row
                 if (fused_scan) {
@@ -983,14 +1012,14 @@ void run_body(mg_model* m, const BodyCtx& c, hipStream_t s) {
                     ring_args(c.sess, ab, r);
                     if (c.sess->kv_packed)
                         HIPCHECK(launch_export_kv_packed(c.B, c.T, D, m->heads, m->cap, c.lens, w.qkv.as<float>(),
-                                                         r.kpack, r.vpack, r.kscale, r.vscale, s));
+                                                         r.kpack, r.vpack, r.kscale, r.vscale, s, c.row0));
                     else
                         HIPCHECK(launch_export_kv(c.B, c.T, D, m->heads, m->cap, c.lens, w.qkv.as<float>(), r.kring,
-                                                  r.vring, s));
+                                                  r.vring, s, c.row0));
                 }
                 AttnArgs aa;
                 aa.B = c.B; aa.T = c.T; aa.D = D; aa.Dp = Dp; aa.heads = m->heads; aa.window = m->window; aa.cap = m->cap;
-                aa.qkv = w.qkv.as<float>(); aa.att = w.att.as<float>();
+                aa.qkv = w.qkv.as<float>(); aa.att = w.att.as<float>(); aa.row0 = c.row0; aa.lens = c.lens;
                 // q, k and v of every position in, the output row out
                 ProfScope ps(m->prof, K_ATTN, s, (double)M * 16.0 * D);
                 HIPCHECK(launch_attention(aa, s));
@@ -1726,9 +1755,34 @@ void generate_sessions_release(mg_model* m, mg_sessions* s) {
 
 namespace {
 
-// Batched prefill on device-resident windowed prompts; leaves the head statistics in ws.
-void prefill_device(mg_sessions* s, const int32_t* prompts_d, const int32_t* lens_d, int max_len, float* logits_d,
-                    HeadCombineArgs hc, hipStream_t st) {
+// Rows of a prefill with its prompts packed, each in whole 16-row tiles, instead of all as long as the longest; 0: not
+// packed. The products, norms and attention of the padding go (400 prompts of 1 to 90 tokens, D256 H512, three blocks,
+// logits to the host: 36000 rows -> 21000, 1860 -> 1477 us; 512 of up to 128, D384 H1024, filled to 31 and to 56 %: 5218 ->
+// 2296 and 5226 -> 3503 us). Against it stands that a packed prefill always takes the scan fused with the rule input, whose
+// rounds of 16 positions run one after another: with few prompts that costs 10 to 35 us per rule step of 128 positions
+// (two prompts of up to 128, D160: 450 -> 574 us). So it is taken where the rows saved are worth it: measured even at
+// about 10000 saved rows x padded state size per padded position (D160: 8600 +3 %, 9800 -4 %; D256: 7700 +7 %, 10500
+// -4 %, 11500 0; D384: 5000 +6 %, 11500 -5 %).
+int prefill_packed_rows(mg_model* m, int S, int Tw, const int32_t* lens, int window) {
+    if (!lens || option(OPT_SCAN_KERNEL) == 1) return 0;
+    for (const DevBlock& blk : m->blocks)
+        for (int st = 0; st < blk.steps; st++)
+            if (!scan_rule_fits(16, m->Dp, blk.dilation(st))) return 0;
+    if (m->nattn) {
+        AttnArgs aa;
+        aa.B = S; aa.T = Tw; aa.D = m->D; aa.Dp = m->Dp; aa.heads = m->heads; aa.window = m->window; aa.cap = m->cap;
+        if (!attention_packs(aa)) return 0;
+    }
+    long long rows = 0;
+    for (int i = 0; i < S; i++) rows += packed_rows(std::min(lens[i], window));
+    const long long saved = (long long)S * Tw - rows;  // more than 0 where packed: the workspace holds S * Tw rows
+    return saved * m->Dp >= 10000LL * Tw ? (int)rows : 0;
+}
+
+// Batched prefill on device-resident windowed prompts; leaves the head statistics in ws. lens_h: the lengths on the host
+// too, or null.
+void prefill_device(mg_sessions* s, const int32_t* prompts_d, const int32_t* lens_d, const int32_t* lens_h, int max_len,
+                    float* logits_d, HeadCombineArgs hc, hipStream_t st) {
     mg_model* m = s->m;
     const int S = s->n;
     const int Tw = std::min(max_len, s->window);
@@ -1737,9 +1791,16 @@ void prefill_device(mg_sessions* s, const int32_t* prompts_d, const int32_t* len
     w.tmp.ensure((size_t)S * Tw * 4);
     int32_t* ids_w = w.tmp.as<int32_t>();
     int32_t* lens_w = w.lens.as<int32_t>();
-    hipLaunchKernelGGL(window_ids_kernel, dim3(S), dim3(128), 0, st, S, max_len, s->window, Tw, prompts_d, lens_d, ids_w, lens_w);
+    const bool seq = seq_usable(m, Tw);
+    const int packed = seq ? 0 : prefill_packed_rows(m, S, Tw, lens_h, s->window);
+    int32_t* row0 = packed ? w.tgt.as<int32_t>() : nullptr;  // (no targets in a prefill)
+    if (packed) {
+        hipLaunchKernelGGL(pack_rows_kernel, dim3(1), dim3(1024), 0, st, S, max_len, s->window, lens_d, row0);
+        HIPCHECK(hipGetLastError());
+    }
+    hipLaunchKernelGGL(window_ids_kernel, dim3(S), dim3(128), 0, st, S, max_len, s->window, Tw, prompts_d, lens_d, row0, ids_w, lens_w);
     HIPCHECK(hipGetLastError());
-    if (seq_usable(m, Tw)) {
+    if (seq) {
         SeqArgs sq = seq_args(m, S, Tw, ids_w);
         sq.lens = lens_w; sq.last_only = true;
         sq.norm_ring = s->norm_ring.as<float>(); sq.g = s->g.as<float>(); sq.ring = m->ring;
@@ -1750,9 +1811,9 @@ void prefill_device(mg_sessions* s, const int32_t* prompts_d, const int32_t* len
         run_head(m, S, nullptr, nullptr, logits_d, hc, st, true);
     } else {
         BodyCtx c;
-        c.B = S; c.T = Tw; c.ids = ids_w; c.sess = s; c.lens = lens_w;
+        c.B = S; c.T = Tw; c.ids = ids_w; c.sess = s; c.lens = lens_w; c.row0 = row0; c.rows = packed;
         run_body(m, c, st);
-        hipLaunchKernelGGL(last_rows_kernel, dim3((S + 255) / 256), dim3(256), 0, st, S, Tw, lens_w, w.rowmap.as<int32_t>());
+        hipLaunchKernelGGL(last_rows_kernel, dim3((S + 255) / 256), dim3(256), 0, st, S, Tw, lens_w, row0, w.rowmap.as<int32_t>());
         HIPCHECK(hipGetLastError());
         run_head(m, S, w.rowmap.as<int32_t>(), nullptr, logits_d, hc, st);
     }
@@ -1921,7 +1982,7 @@ int mg_sessions_prefill(mg_sessions* s, const int32_t* prompts, const int32_t* l
         HeadCombineArgs hc;
         hc.argmax = argmax ? (dev ? argmax : sg.out<int32_t>(S)) : nullptr;
         hc.prob = prob ? (dev ? prob : sg.out<double>(S)) : nullptr;
-        prefill_device(s, p_d, l_d, max_len, lg, hc, st);
+        prefill_device(s, p_d, l_d, dev ? nullptr : lens, max_len, lg, hc, st);
         if (!dev) {
             if (logits) HIPCHECK(hipMemcpyAsync(logits, lg, (size_t)S * m->V * 4, hipMemcpyDeviceToHost, st));
             if (argmax) HIPCHECK(hipMemcpyAsync(argmax, hc.argmax, (size_t)S * 4, hipMemcpyDeviceToHost, st));
@@ -2123,7 +2184,7 @@ int mg_sessions_decode_greedy(mg_sessions* s, const int32_t* prompts, const int3
         HeadCombineArgs hc;
         hc.next_ids = s->next_ids.as<int32_t>();
         hc.out_ids = oi; hc.out_probs = op; hc.out_ld = max_tokens; hc.out_col = 0;
-        prefill_device(s, p_d, l_d, max_len, nullptr, hc, st);
+        prefill_device(s, p_d, l_d, dev ? nullptr : lens, max_len, nullptr, hc, st);
         hc.col = start_columns(s, st);
         int k = 1;
         for (; k + kStepsPerGraph <= max_tokens; k += kStepsPerGraph)
@@ -2169,7 +2230,7 @@ int mg_sessions_decode_greedy_until(mg_sessions* s, const int32_t* prompts, cons
         HeadCombineArgs hc;
         hc.next_ids = s->next_ids.as<int32_t>();
         hc.out_ids = oi; hc.out_probs = op; hc.out_ld = max_tokens; hc.out_col = 0;
-        prefill_device(s, p_d, l_d, max_len, nullptr, hc, st);
+        prefill_device(s, p_d, l_d, dev ? nullptr : lens, max_len, nullptr, hc, st);
         tr.scan(0);
         const bool first = tr.keep_going(0);  // false: cancelled before the first token
         hc.col = start_columns(s, st);
@@ -2239,7 +2300,7 @@ int mg_sessions_decode_sample(mg_sessions* s, const int32_t* prompts, const int3
             tr.scan(col);
         };
         HeadCombineArgs hc;  // the sampler, not the argmax, picks each token
-        prefill_device(s, p_d, l_d, max_len, lg, hc, st);
+        prefill_device(s, p_d, l_d, dev ? nullptr : lens, max_len, lg, hc, st);
         pick(0);
         const bool first = tr.keep_going(0);  // false: cancelled before the first token
         if (n_stops > 0) hc.done = tr.cnt;  // sessions past their stop token need no further steps

@@ -405,7 +405,8 @@ template <bool RN>
 __global__ __launch_bounds__(512) void scan_rule_kernel(ScanArgs a) {
     extern __shared__ __align__(16) int8_t sr_smem[];
     const int b = blockIdx.x, j = threadIdx.x, lane = j & 63, w = j >> 6, nw = blockDim.x >> 6;
-    const int D = a.D, Dp = a.Dp, T = a.T, C2 = Dp >> 1, dil = a.dil;
+    const int D = a.D, Dp = a.Dp, C2 = Dp >> 1, dil = a.dil;
+    const int T = a.row0 ? packed_rows(a.lens[b]) : a.T;
     const int jc = min(j, C2 - 1);
     const int seg_bytes = (Dp >> 6) * 3072;  // one segment of a tile: Dp/64 K steps x 3 limbs x 1 KiB
     int8_t* stage = sr_smem;
@@ -413,7 +414,7 @@ __global__ __launch_bounds__(512) void scan_rule_kernel(ScanArgs a) {
     float* nring = red + 32 * nw;                                // [64] max|n| of row t at t & 63
     float* part = nring + 64;                                    // [16] max(|n|, |g|) of the round's rows
     float* invs = part + 16;                                     // [16] 127 / row absmax
-    const long long seq0 = (long long)b * T;
+    const long long seq0 = a.row0 ? a.row0[b] : (long long)b * T;
     const int last = a.lens ? a.lens[b] - 1 : -1;
     const bool on = j < C2;
     const bool c0 = on && 2 * j < D, c1 = on && 2 * j + 1 < D;  // columns past D are zero
@@ -895,16 +896,19 @@ __global__ __launch_bounds__(64 * G) void attention_mfma_kernel(AttnArgs a, int 
     constexpr int PER = (NCH + NT - 1) / NT;
     extern __shared__ __align__(16) float att_lds[];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, tid = threadIdx.x;
-    const int T = a.T, D = a.D, cap = a.cap, ld = 3 * D;
-    const int qtiles = (T + 15) >> 4;
-    const int groups = (qtiles + G - 1) / G;
+    const int D = a.D, cap = a.cap, ld = 3 * D;
+    const int groups = (((a.T + 15) >> 4) + G - 1) / G;
     const int b = blockIdx.x / groups;
     const int grp = blockIdx.x % groups;
+    const int T = a.row0 ? packed_rows(a.lens[b]) : a.T;
+    const int qtiles = (T + 15) >> 4;
+    if (grp * G >= qtiles) return;  // (packed sequences) past this one's end, the whole workgroup
+    const long long seq0 = a.row0 ? a.row0[b] : (long long)b * T;
     const int tile = grp * G + w;
     const int h = blockIdx.y;
     const int t0 = tile * 16;
     const int qi = lane & 15, kg = lane >> 4;
-    const float* seq = a.qkv + (long long)b * T * ld;
+    const float* seq = a.qkv + seq0 * ld;
     const float* qb = seq + h * dh;
     const float* kb_ = seq + D + h * dh;
     const float* vb = seq + 2 * D + h * dh;
@@ -1015,7 +1019,7 @@ __global__ __launch_bounds__(64 * G) void attention_mfma_kernel(AttnArgs a, int 
     for (int r = 0; r < 4; r++) {
         const int tq = t0 + 4 * kg + r;
         if (tq >= T) continue;
-        float* dst = a.att + ((long long)b * T + tq) * a.Dp + h * dh;
+        float* dst = a.att + (seq0 + tq) * a.Dp + h * dh;
 #pragma unroll
         for (int g = 0; g < ND; g++) {
             const int d = 16 * g + qi;
@@ -3084,26 +3088,30 @@ __global__ void quantize_kernel(const float* w, long long n, int8_t* q, const un
 // ------------------------------------------------------------------------------------------------
 // session state export and small helpers
 // ------------------------------------------------------------------------------------------------
-__global__ void export_ring_kernel(int B, int T, int Dp, int ring, const int32_t* lens, const float* nf, float* nr) {
+// row0: each sequence's first row (packed sequences), or null: b * T.
+__global__ void export_ring_kernel(int B, int T, int Dp, int ring, const int32_t* lens, const float* nf, float* nr,
+                                   const int32_t* row0) {
     const int b = blockIdx.x;
     const int len = lens[b];
     const int p0 = max(0, len - ring);
+    const long long seq0 = row0 ? row0[b] : (long long)b * T;
     for (int p = p0; p < len; p++)
         for (int d = threadIdx.x; d < Dp; d += blockDim.x)
-            nr[((long long)b * ring + p % ring) * Dp + d] = nf[((long long)b * T + p) * Dp + d];
+            nr[((long long)b * ring + p % ring) * Dp + d] = nf[(seq0 + p) * Dp + d];
 }
 
 // The rings are head-major, [session][head][slot][dh], so that a decode step's key and value rows of one
 // head are one contiguous block.
 __global__ void export_kv_kernel(int B, int T, int D, int heads, int cap, const int32_t* lens, const float* qkv,
-                                 float* kr, float* vr) {
+                                 float* kr, float* vr, const int32_t* row0) {
     const int b = blockIdx.x;
     const int len = min(max(lens[b], 0), T);
     const int p0 = max(0, len - cap);
+    const long long seq0 = row0 ? row0[b] : (long long)b * T;
     const int dh = D / heads;
     for (int p = p0; p < len; p++)
         for (int d = threadIdx.x; d < D; d += blockDim.x) {
-            const float* row = qkv + ((long long)b * T + p) * 3 * D;
+            const float* row = qkv + (seq0 + p) * 3 * D;
             const int h = d / dh;
             const long long o = (((long long)b * heads + h) * cap + p % cap) * dh + (d - h * dh);
             kr[o] = row[D + d];
@@ -3119,16 +3127,18 @@ __host__ __device__ inline int export_kv_wave_floats(int D, int heads) { return 
 
 __global__ __launch_bounds__(256) void export_kv_packed_kernel(int B, int T, int D, int heads, int cap,
                                                                const int32_t* lens, const float* qkv, uint32_t* kpack,
-                                                               uint32_t* vpack, float* kscale, float* vscale) {
+                                                               uint32_t* vpack, float* kscale, float* vscale,
+                                                               const int32_t* row0) {
     extern __shared__ __align__(16) float ex_smem[];
     const int b = blockIdx.x, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int len = min(max(lens[b], 0), T);
     const int p0 = max(0, len - cap);
+    const long long seq0 = row0 ? row0[b] : (long long)b * T;
     const int dh = D / heads, c4 = dh / 4, nc = D / 2;  // float4 chunks of [k | v]
     float* xw = ex_smem + w * export_kv_wave_floats(D, heads);
     int* ew = (int*)(xw + 2 * D);  // [2 heads] row exponents: rows 0..heads-1 keys, heads..2heads-1 values
     for (int p = p0 + w; p < len; p += 4) {
-        const float* src = qkv + ((long long)b * T + p) * 3 * D + D;  // k then v, 2D floats
+        const float* src = qkv + (seq0 + p) * 3 * D + D;  // k then v, 2D floats
         for (int c = lane; c < nc; c += 64) *(float4*)(xw + 4 * c) = ldg((const float4*)(src + 4 * c));
         wave_lds_sync();
         for (int r = lane; r < 2 * heads; r += 64) {
@@ -3155,16 +3165,17 @@ template <int C4>
 __global__ __launch_bounds__(256) void export_kv_packed_dpp_kernel(int B, int T, int D, int heads, int cap,
                                                                    const int32_t* lens, const float* qkv,
                                                                    uint32_t* kpack, uint32_t* vpack, float* kscale,
-                                                                   float* vscale) {
+                                                                   float* vscale, const int32_t* row0) {
     const int b = blockIdx.x, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int len = min(max(lens[b], 0), T);
     const int p0 = max(0, len - cap);
+    const long long seq0 = row0 ? row0[b] : (long long)b * T;
     const int nc = D / 2;                        // groups of [k | v] per position
     const int per = (nc + 63) / 64;              // 64-lane passes per position
     for (int it = w; it < (len - p0) * per; it += 4) {
         const int p = p0 + it / per, c = (it % per) * 64 + lane;
         const bool ok = c < nc;
-        const float4 x = ldg((const float4*)(qkv + ((long long)b * T + p) * 3 * D + D + 4 * min(c, nc - 1)));
+        const float4 x = ldg((const float4*)(qkv + (seq0 + p) * 3 * D + D + 4 * min(c, nc - 1)));
         float m = fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w)));
         if constexpr (C4 >= 2) m = fmaxf(m, dpp_move<0xB1>(m));   // quad_perm [1, 0, 3, 2]
         if constexpr (C4 >= 4) m = fmaxf(m, dpp_move<0x4E>(m));   // quad_perm [2, 3, 0, 1]
@@ -3443,7 +3454,7 @@ hipError_t launch_scan(const ScanArgs& a, hipStream_t s) {
 bool scan_rule_fits(int T, int Dp, int dil) { return T % 16 == 0 && Dp % 64 == 0 && Dp <= 1024 && dil >= 1 && dil <= 48; }
 
 hipError_t launch_scan_rule(const ScanArgs& a, hipStream_t s) {
-    if (!scan_rule_fits(a.T, a.Dp, a.dil) || a.D > a.Dp) return hipErrorInvalidValue;
+    if (!scan_rule_fits(a.row0 ? 16 : a.T, a.Dp, a.dil) || a.D > a.Dp || (a.row0 && !a.lens)) return hipErrorInvalidValue;
     if (a.B == 0 || a.T == 0) return hipSuccess;
     const int threads = ((a.Dp / 2 + 63) / 64) * 64;
     const size_t lds = (size_t)(a.Dp / 64) * 3 * 1088 + (2 * (threads / 64) * 16 + 64 + 16 + 16) * sizeof(float);
@@ -3490,9 +3501,14 @@ bool dh_compiled(int dh) {
     }
 }
 
+bool attention_packs(const AttnArgs& a) {
+    return a.heads > 0 && a.D % a.heads == 0 && a.cap > 0 && option(OPT_ATTENTION_KERNEL) != ATTN_EXACT &&
+           attn_mfma_fits(a, a.D / a.heads);
+}
+
 hipError_t launch_attention(const AttnArgs& a, hipStream_t s) {
     if (a.B <= 0 || a.T <= 0) return hipSuccess;
-    if (a.heads <= 0 || a.D % a.heads || a.cap <= 0) return hipErrorInvalidValue;
+    if (a.heads <= 0 || a.D % a.heads || a.cap <= 0 || (a.row0 && (!a.lens || !attention_packs(a)))) return hipErrorInvalidValue;
     const int dh = a.D / a.heads;
     const int mode = option(OPT_ATTENTION_KERNEL);
     if (mode != ATTN_EXACT && attn_mfma_fits(a, dh)) return attn_mfma(a, dh, s);
@@ -3670,22 +3686,22 @@ hipError_t launch_quantize(const float* w, long long n, int8_t* q, float* scale,
 }
 
 hipError_t launch_export_ring(int B, int T, int Dp, int ring, const int32_t* lens, const float* nf, float* norm_ring,
-                              hipStream_t s) {
+                              hipStream_t s, const int32_t* row0) {
     if (B <= 0) return hipSuccess;
-    hipLaunchKernelGGL(export_ring_kernel, dim3(B), dim3(256), 0, s, B, T, Dp, ring, lens, nf, norm_ring);
+    hipLaunchKernelGGL(export_ring_kernel, dim3(B), dim3(256), 0, s, B, T, Dp, ring, lens, nf, norm_ring, row0);
     return hipGetLastError();
 }
 
 hipError_t launch_export_kv(int B, int T, int D, int heads, int cap, const int32_t* lens, const float* qkv,
-                            float* kring, float* vring, hipStream_t s) {
+                            float* kring, float* vring, hipStream_t s, const int32_t* row0) {
     if (B <= 0) return hipSuccess;
     if (heads <= 0 || D % heads != 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(export_kv_kernel, dim3(B), dim3(256), 0, s, B, T, D, heads, cap, lens, qkv, kring, vring);
+    hipLaunchKernelGGL(export_kv_kernel, dim3(B), dim3(256), 0, s, B, T, D, heads, cap, lens, qkv, kring, vring, row0);
     return hipGetLastError();
 }
 
 hipError_t launch_export_kv_packed(int B, int T, int D, int heads, int cap, const int32_t* lens, const float* qkv,
-                                   uint32_t* kpack, uint32_t* vpack, float* kscale, float* vscale, hipStream_t s) {
+                                   uint32_t* kpack, uint32_t* vpack, float* kscale, float* vscale, hipStream_t s, const int32_t* row0) {
     if (B <= 0) return hipSuccess;
     if (heads <= 0 || D % heads != 0 || (D / heads) % 4) return hipErrorInvalidValue;
     if (D > 1024) return hipErrorInvalidValue;
@@ -3693,7 +3709,7 @@ hipError_t launch_export_kv_packed(int B, int T, int D, int heads, int cap, cons
 #define MG_EXPORT_DPP(C)                                                                                        \
     case C:                                                                                                     \
         hipLaunchKernelGGL(export_kv_packed_dpp_kernel<C>, dim3(B), dim3(256), 0, s, B, T, D, heads, cap, lens, qkv, \
-                           kpack, vpack, kscale, vscale);                                                       \
+                           kpack, vpack, kscale, vscale, row0);                                                 \
         return hipGetLastError();
         MG_EXPORT_DPP(1)
         MG_EXPORT_DPP(2)
@@ -3705,7 +3721,7 @@ hipError_t launch_export_kv_packed(int B, int T, int D, int heads, int cap, cons
     }
     const size_t lds = (size_t)4 * export_kv_wave_floats(D, heads) * sizeof(float);
     hipLaunchKernelGGL(export_kv_packed_kernel, dim3(B), dim3(256), lds, s, B, T, D, heads, cap, lens, qkv, kpack,
-                       vpack, kscale, vscale);
+                       vpack, kscale, vscale, row0);
     return hipGetLastError();
 }
 

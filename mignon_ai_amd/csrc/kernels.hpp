@@ -6,6 +6,9 @@
 
 namespace mg {
 
+// Rows of a packed sequence: whole 16-row tiles.
+__host__ __device__ inline int packed_rows(int len) { return (len + 15) & ~15; }
+
 enum RowMode : int { ROW_SRC = 0, ROW_EMBED = 1, ROW_RESID = 2, ROW_RULE = 3 };
 
 // Values of OPT_ATTENTION_KERNEL.
@@ -49,6 +52,8 @@ struct ScanArgs {
     float* g = nullptr;          // [B*T][Dp] latch state after each position (may be lam itself)
     const int32_t* lens = nullptr;  // per-sequence length (export position lens[b]-1) or null
     float* g_out = nullptr;         // exported latch state [B][Dp] or null
+    // scan_rule only: packed sequences (with lens): sequence b is packed_rows(lens[b]) rows from row0[b] on
+    const int32_t* row0 = nullptr;
     // scan_rule only: the rule input [n | left | g] limb-expanded (K = 3*Dp) with one scale per row
     int dil = 1;
     int8_t* xl = nullptr;
@@ -77,7 +82,12 @@ struct AttnArgs {
     int B = 0, T = 0, D = 0, Dp = 0, heads = 0, window = 0, cap = 0;
     const float* qkv = nullptr;  // [B*T][3D]
     float* att = nullptr;        // [B*T][Dp]
+    // packed sequences of at most T rows (attention_packs): sequence b is packed_rows(lens[b]) rows from row0[b] on
+    const int32_t* row0 = nullptr;
+    const int32_t* lens = nullptr;
 };
+// Whether launch_attention takes packed sequences at these sizes.
+bool attention_packs(const AttnArgs& a);
 hipError_t launch_attention(const AttnArgs& a, hipStream_t s);
 
 // The attention projection fused with windowed attention (teacher-forced forward): per sequence and head,
@@ -246,12 +256,12 @@ hipError_t launch_quantize(const float* w, long long n, int8_t* q, float* scale,
 
 // Session state export after a batched prefill.
 hipError_t launch_export_ring(int B, int T, int Dp, int ring, const int32_t* lens, const float* nf, float* norm_ring,
-                              hipStream_t s);
+                              hipStream_t s, const int32_t* row0 = nullptr);
 hipError_t launch_export_kv(int B, int T, int D, int heads, int cap, const int32_t* lens, const float* qkv,
-                            float* kring, float* vring, hipStream_t s);
+                            float* kring, float* vring, hipStream_t s, const int32_t* row0 = nullptr);
 // The same into packed rings (AttnStepArgs::kpack's layout; head width a multiple of 4).
 hipError_t launch_export_kv_packed(int B, int T, int D, int heads, int cap, const int32_t* lens, const float* qkv,
-                                   uint32_t* kpack, uint32_t* vpack, float* kscale, float* vscale, hipStream_t s);
+                                   uint32_t* kpack, uint32_t* vpack, float* kscale, float* vscale, hipStream_t s, const int32_t* row0 = nullptr);
 // pos[i] = (lens ? lens[i] : pos[i]) + add; with col set, also advances the decode column *col by one.
 hipError_t launch_set_pos(int S, const int32_t* lens, int32_t* pos, int add, hipStream_t s, int32_t* col = nullptr);
 hipError_t launch_fill_i32(int32_t* p, int n, int v, hipStream_t s);
