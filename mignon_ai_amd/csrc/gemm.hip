@@ -1008,7 +1008,7 @@ __global__ __launch_bounds__(256) void gemm_c2_kernel(GemmArgs g) {
     __shared__ __align__(16) int8_t Ws[2][GEMM_BN * LDSR];
     __shared__ __align__(16) int8_t As[2][GEMM_BM * LDSR];
 
-    const int nt = (g.Np + GEMM_BN - 1) / GEMM_BN;
+    const int nt = RAGGED ? (g.Np + GEMM_BN - 1) / GEMM_BN : g.Np / GEMM_BN;
     const int mt = (g.M + GEMM_BM - 1) / GEMM_BM;
     const int total = nt * mt;
     const int t = xcd_tile(blockIdx.x, total);
@@ -1058,7 +1058,7 @@ __global__ __launch_bounds__(256) void gemm_c2_kernel(GemmArgs g) {
 #pragma unroll
         for (int tj = 0; tj < 2; tj++) acc[ti][tj] = v4i{0, 0, 0, 0};
 
-    const int ksteps = (g.Kp + GEMM_BK - 1) / GEMM_BK;
+    const int ksteps = RAGGED ? (g.Kp + GEMM_BK - 1) / GEMM_BK : g.Kp / GEMM_BK;
     gload(0);
     sstore(0);
     __syncthreads();
