@@ -1763,7 +1763,7 @@ namespace {
 // (two prompts of up to 128, D160: 450 -> 574 us). So it is taken where the rows saved are worth it: measured even at
 // about 10000 saved rows x padded state size per padded position (D160: 8600 +3 %, 9800 -4 %; D256: 7700 +7 %, 10500
 // -4 %, 11500 0; D384: 5000 +6 %, 11500 -5 %).
-int prefill_packed_rows(mg_model* m, int S, int Tw, const int32_t* lens, int window) {
+int prefill_packed_rows(mg_model* m, int S, int max_len, int Tw, const int32_t* lens, int window) {
     if (!lens || option(OPT_SCAN_KERNEL) == 1) return 0;
     for (const DevBlock& blk : m->blocks)
         for (int st = 0; st < blk.steps; st++)
@@ -1774,7 +1774,7 @@ int prefill_packed_rows(mg_model* m, int S, int Tw, const int32_t* lens, int win
         if (!attention_packs(aa)) return 0;
     }
     long long rows = 0;
-    for (int i = 0; i < S; i++) rows += packed_rows(std::min(lens[i], window));
+    for (int i = 0; i < S; i++) rows += packed_rows(std::min(std::min(std::max(lens[i], 1), max_len), window));
     const long long saved = (long long)S * Tw - rows;  // more than 0 where packed: the workspace holds S * Tw rows
     return saved * m->Dp >= 10000LL * Tw ? (int)rows : 0;
 }
@@ -1792,7 +1792,7 @@ void prefill_device(mg_sessions* s, const int32_t* prompts_d, const int32_t* len
     int32_t* ids_w = w.tmp.as<int32_t>();
     int32_t* lens_w = w.lens.as<int32_t>();
     const bool seq = seq_usable(m, Tw);
-    const int packed = seq ? 0 : prefill_packed_rows(m, S, Tw, lens_h, s->window);
+    const int packed = seq ? 0 : prefill_packed_rows(m, S, max_len, Tw, lens_h, s->window);
     int32_t* row0 = packed ? w.tgt.as<int32_t>() : nullptr;  // (no targets in a prefill)
     if (packed) {
         hipLaunchKernelGGL(pack_rows_kernel, dim3(1), dim3(1024), 0, st, S, max_len, s->window, lens_d, row0);
