@@ -15,7 +15,8 @@
 // Activations are expanded to three base-256 digits with one scale per row (scale = amax / 127, digits of
 // round(x * 127 * 65536 / amax): 0.5 / 8323072 of the row's maximum, the limb planes' own resolution).
 //
-// Weights are read once per workgroup, as a stream of units of UF fragments (1 KiB each) in the order of use, moved
+// Weights are read by the workgroup as a stream of units of UF fragments (1 KiB each) in the order of use (a block's rule
+// steps read the same units again, so that the stream is no longer than the weights whatever the step count), moved
 // straight from memory into four LDS slots: while unit u is used, units u + 1 to u + 3 are on their way, one barrier a
 // unit. A unit takes 1 to 2 thousand cycles and a load that misses the L2 about two thousand, so with only one unit
 // between a request and its use (through registers, two slots) every unit waited some 500 cycles: 1024 x 128 tokens of
@@ -82,12 +83,13 @@ __device__ __forceinline__ void wg_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// One 16-byte load per lane from global memory straight into LDS: lane L's bytes land at LDS offset lds + 16 L. Inline
-// assembly, with the waits written out (vm_wait), because the compiler would wait for all such loads before any LDS read.
-// The LDS address goes through M0, which nothing else in this file's device code uses; the s_nop is the wait state
-// between the write of M0 and its use. No register receives anything.
-__device__ __forceinline__ void lds_load16(const void* g, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds) : "memory");
+// One 16-byte load per lane from global memory straight into LDS: lane L reads base + off and its bytes land at LDS offset
+// lds + 16 L. Inline assembly, with the waits written out (vm_wait), because the compiler would wait for all such loads
+// before any LDS read. The LDS address goes through M0. The base is a scalar register pair: a vector instruction may have
+// written it (the compiler keeps spilled scalars in vector lanes), which takes five wait states before a memory instruction
+// reads it, and one between the write of M0 and its use: the move counts one, the s_nop four. No register receives anything.
+__device__ __forceinline__ void lds_load16(const int8_t* base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
 }
 __device__ __forceinline__ uint32_t lds_offset(const void* p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
@@ -293,12 +295,13 @@ __global__ __launch_bounds__(512)
     const bool key_act = in_rows && 16 * tile + 15 >= rows.x - span + 1;
 
     // The weight stream: wave w moves fragments w and w + 8 of every unit, unit u to LDS slot u & 3.
-    const int8_t* wp = a.stream + w * 1024 + lane * 16;
+    const int8_t* wp = a.stream + w * 1024;
+    const uint32_t wlane = lane * 16;
     const uint32_t slots = lds_offset(smem) + w * 1024;
     auto request = [&](int u) {
         const uint32_t d = slots + (u & (kSlots - 1)) * (C::UF * 1024);
-        if (C::UF >= 8 || w < C::UF) lds_load16(wp, d);
-        if (C::UF > 8 && w + 8 < C::UF) lds_load16(wp + 8192, d + 8192);
+        if (C::UF >= 8 || w < C::UF) lds_load16(wp, wlane, d);
+        if (C::UF > 8 && w + 8 < C::UF) lds_load16(wp + 8192, wlane, d + 8192);
         wp += C::UF * 1024;
     };
     // this wave's fragments of all units but the `newer` last requested have arrived
@@ -341,6 +344,12 @@ __global__ __launch_bounds__(512)
         idle_units(DT);
     };
     constexpr int RULE2 = 4 * HT + 4 * DT / C::HW;  // units of a rule step after the latch's DT
+    constexpr int RULE = DT + RULE2;
+    // A block's rule steps share one copy of their units: before the request of the unit past a step's last (made three
+    // units ahead, at the step's unit RULE - 3), the stream goes back to the step's first unit if another step follows.
+    constexpr int TURN = RULE - (kSlots - 1);
+    static_assert(TURN >= DT, "the turn lies among the units after the latch's");
+    auto turn = [&](bool again) { wp -= again ? RULE * C::UF * 1024 : 0; };
 
     // out-of-range ids are token 0, as are the positions past the sequence
     int id = mine && t < a.T ? a.ids[(long long)b * a.T + t] : 0;
@@ -351,7 +360,11 @@ __global__ __launch_bounds__(512)
         arrived(std::integral_constant<int, kSlots - 2>{});
         wg_barrier();
         for (int blk = 0; blk < a.nblocks; blk++) {
-            idle_units(a.blocks[blk].steps * (DT + RULE2));
+            for (int st = 1; st <= a.blocks[blk].steps; st++) {
+                idle_units(TURN);
+                turn(st < a.blocks[blk].steps);
+                idle_units(RULE - TURN);
+            }
             if (ND > 0 && a.blocks[blk].attn) idle_attention();
             if (blk + 1 < a.nblocks) {
                 vec_load(blk + 1);
@@ -538,6 +551,7 @@ __global__ __launch_bounds__(512)
             };
 #pragma unroll
             for (int p = 0; p < 4 * HT; p++) {
+                if (DT + p == TURN) turn(st + 1 < steps);
                 const int8_t* wl = begin();
                 if (p > 0) {
                     float bv[4], bg[4];
@@ -589,6 +603,7 @@ __global__ __launch_bounds__(512)
             Vecs vlast[C::HW];
 #pragma unroll
             for (int un = 0; un < NU; un++) {
+                if (DT + 4 * HT + un == TURN) turn(st + 1 < steps);
                 const int8_t* wl = begin();
                 if (un > 0) {
                     Vecs vs[C::HW];
@@ -919,7 +934,7 @@ SeqPack seq_pack(const HostModel& hm, SeqShape sh, const std::vector<float>& lat
         b.attn = hb.has_attn ? 1 : 0; b.norm = (int)hb.gamma.size() == D ? 1 : 0;
         b.ssel = hb.ssel; b.s1 = hb.s1; b.s2 = hb.s2; b.sqkv = hb.sqkv; b.so = hb.so;
         p.blocks.push_back(b);
-        for (int st = 0; st < hb.steps; st++) {
+        if (hb.steps > 0) {  // one copy, read again by every step
             for (int un = 0; un < DT; un++) {
                 open();
                 for (int ks = 0; ks < DT; ks++)

@@ -29,7 +29,7 @@ struct SeqShape {
 // span: keys a position attends at most.
 SeqShape seq_shape(const HostModel& hm, int span);
 
-// The weights in the order the kernel reads them, and the vectors [latch base | per block b1 | b2 | gamma |
+// The weights in the order the kernel reads them (each block's rule units once), and the vectors [latch base | per block b1 | b2 | gamma |
 // attention gamma] it copies to LDS block by block.
 struct SeqPack {
     std::vector<int8_t> stream;

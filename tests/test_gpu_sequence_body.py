@@ -10,6 +10,7 @@ from mignon_ai_amd import Model, engine_option, synth
 from mignon_ai_amd.evaluate import score_sequences
 
 pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
 
 # D, H, heads, window, blocks: one entry per compiled variant, among them head widths of no whole groups of four or
 # below 16, several rule steps with dilations up to 32, a block without steps, windows of one key and of a whole tile
@@ -121,3 +122,27 @@ def test_forward_many_sequences():
     assert rel_err(got[:, :-1], want[:, :-1]).max() < 2e-5
     sub = [0, 599]
     assert_close(Model(data).forward_batch(ids[sub])["logits"], oracle_model(data).forward_all(ids[sub]), what="c3")
+
+
+def test_many_steps():
+    """A block's rule steps share one copy of the kernel's weights: a file of many steps loads in the memory of its
+    weights, and repeated steps, waves without work among them, equal the layered body."""
+    spec = tiny_spec([(20000, 2, 1)], V=131, D=32, H=64, context=128)
+    data = uniform_model_bytes(spec, seed=6, scale=0.3)
+    free = torch.cuda.mem_get_info()[0]
+    m = Model(data)
+    used = free - torch.cuda.mem_get_info()[0]
+    assert used < 64 << 20, used  # its 20000 copies would be 20000 steps x 7 units x 6 KiB = 820 MiB
+    del m
+    ids = synth.token_ids(78, "steps", (11, 70), 131)
+    lens = np.array([1, 70, 17, 33, 40, 16, 69, 2, 50, 64, 65], np.int32)
+    for D, H, heads, blocks in ((32, 64, 0, [(7, 2, 1), (5, 2, 1)]), (128, 256, 4, [(3, 2, 1), (9, 2, 2), (6, 2, 1)])):
+        spec = tiny_spec(blocks, V=131, D=D, H=H, heads=heads, window=64 if heads else 0, context=128, tied=False)
+        m = Model(uniform_model_bytes(spec, seed=7, scale=0.25))
+        out = {}
+        for mode in ("auto", "limbs"):
+            engine_option("operands", mode)
+            s = m.sessions(len(ids), 128)
+            out[mode] = m.forward_batch(ids)["logits"], s.prefill(ids, lens)[0], s.step(ids[:, 0])[0]
+        for a, b in zip(out["auto"], out["limbs"]):
+            assert_close(a, b, rtol=2e-5, what=f"{blocks}")
