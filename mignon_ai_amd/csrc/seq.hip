@@ -89,7 +89,7 @@ __device__ __forceinline__ void wg_barrier() {
 // written it (the compiler keeps spilled scalars in vector lanes), which takes five wait states before a memory instruction
 // reads it, and one between the write of M0 and its use: the move counts one, the s_nop four. No register receives anything.
 __device__ __forceinline__ void lds_load16(const int8_t* base, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "m0", "memory");
 }
 __device__ __forceinline__ uint32_t lds_offset(const void* p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
