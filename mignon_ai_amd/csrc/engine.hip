@@ -122,8 +122,15 @@ struct PinnedIO {
     void ensure(size_t in, size_t out) {
         if (host) return;
         in = (in + 255) / 256 * 256;
-        HIPCHECK(hipHostMalloc((void**)&host, in + out, hipHostMallocCoherent | hipHostMallocMapped));
-        HIPCHECK(hipHostGetDevicePointer((void**)&dev, host, 0));
+        void* h = nullptr;
+        void* d = nullptr;
+        HIPCHECK(hipHostMalloc(&h, in + out, hipHostMallocCoherent | hipHostMallocMapped));
+        if (const hipError_t e = hipHostGetDevicePointer(&d, h, 0); e != hipSuccess) {
+            (void)hipHostFree(h);  // or the next call would take the region without its device address
+            HIPCHECK(e);
+        }
+        host = (uint8_t*)h;
+        dev = (uint8_t*)d;
         in_bytes = in;
     }
 };
