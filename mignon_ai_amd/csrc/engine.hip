@@ -127,7 +127,7 @@ struct PinnedIO {
         HIPCHECK(hipHostMalloc(&h, in + out, hipHostMallocCoherent | hipHostMallocMapped));
         if (const hipError_t e = hipHostGetDevicePointer(&d, h, 0); e != hipSuccess) {
             (void)hipHostFree(h);  // or the next call would take the region without its device address
-            HIPCHECK(e);
+            hip_check(e, "hipHostGetDevicePointer");
         }
         host = (uint8_t*)h;
         dev = (uint8_t*)d;
