@@ -1045,8 +1045,8 @@ void run_body(mg_model* m, const BodyCtx& c, hipStream_t s) {
 }
 
 // The same body for B sequences of T tokens in one kernel (seq.hip), which leaves the head's operand in ws.nl / ws.ns:
-// the final-normalised rows of the positions `rows` names (null: all), where it takes the model and the length. Any
-// engine option that selects one of the layered kernels selects the layered body.
+// the final-normalised rows of the positions `rows` names (null: all), where it takes the model and the length and is the
+// faster body for that many sequences. Any engine option that selects one of the layered kernels selects the layered body.
 SeqArgs seq_args(mg_model* m, int B, int T, const int32_t* ids) {
     Workspace& w = ws_of(m);
     SeqArgs a;
@@ -1058,11 +1058,11 @@ SeqArgs seq_args(mg_model* m, int B, int T, const int32_t* ids) {
     return a;
 }
 
-bool seq_usable(mg_model* m, int T) {
+bool seq_usable(mg_model* m, int B, int T) {
     if (option(OPT_GEMM_KERNEL) || option(OPT_ATTENTION_KERNEL) || option(OPT_SCAN_KERNEL) || option(OPT_OPERANDS)) return false;
     SeqArgs a;
-    a.shape = m->seq_shape; a.B = 1; a.T = T;
-    return seq_fits(a);
+    a.shape = m->seq_shape; a.B = B; a.T = T;
+    return seq_fits(a) && seq_pays(a.shape, B, T, m->nbs, m->nattn, m->heads);
 }
 
 void run_seq(mg_model* m, const SeqArgs& a, hipStream_t s) {
@@ -1488,7 +1488,7 @@ int mg_forward_batch(mg_model* m, const int32_t* ids, int B, int T, float* logit
             int32_t* ids_d = w.ids.as<int32_t>();
             if (dev) HIPCHECK(hipMemcpyAsync(ids_d, ids + row0, (size_t)M * 4, hipMemcpyDeviceToDevice, s));
             else HIPCHECK(hipMemcpyAsync(ids_d, ids + row0, (size_t)M * 4, hipMemcpyHostToDevice, s));
-            const bool seq = seq_usable(m, T);
+            const bool seq = seq_usable(m, Bc, T);
             {
                 ProfScope ps(m->prof, K_ROW, s, (double)M * 8.0);
                 hipLaunchKernelGGL(targets_kernel, dim3((M + 255) / 256), dim3(256), 0, s, M, T, ids_d, w.tgt.as<int32_t>());
@@ -1601,7 +1601,7 @@ int mg_score_sequences(mg_model* m, const int32_t* tokens, const long long* offs
             const size_t r1 = std::min(rows.size(), r0 + (size_t)(cap / T));
             const int B = (int)(r1 - r0);
             h_start.clear(); h_len.clear(); h_map.clear(); h_tgt.clear(); h_rows.clear();
-            const bool seq = seq_usable(m, T);  // the one-kernel body computes the scored positions' rows only
+            const bool seq = seq_usable(m, B, T);  // the one-kernel body computes the scored positions' rows only
             for (size_t r = r0; r < r1; r++) {
                 const Row& row = rows[r];
                 h_start.push_back(row.start);
@@ -1665,7 +1665,7 @@ int mg_model_call(mg_model* m, const int32_t* ids, int n, double* logits) {
         const int32_t* ids_d = (const int32_t*)m->call_io.dev;
         float* lg = (float*)(m->call_io.dev + m->call_io.in_bytes);
         HeadCombineArgs hc;
-        if (seq_usable(m, n)) {
+        if (seq_usable(m, 1, n)) {
             SeqArgs sq = seq_args(m, 1, n, ids_d);
             sq.last_only = true;
             run_seq(m, sq, s);
@@ -1798,7 +1798,7 @@ void prefill_device(mg_sessions* s, const int32_t* prompts_d, const int32_t* len
     w.tmp.ensure((size_t)S * Tw * 4);
     int32_t* ids_w = w.tmp.as<int32_t>();
     int32_t* lens_w = w.lens.as<int32_t>();
-    const bool seq = seq_usable(m, Tw);
+    const bool seq = seq_usable(m, S, Tw);
     const int packed = seq ? 0 : prefill_packed_rows(m, S, max_len, Tw, lens_h, s->window);
     int32_t* row0 = packed ? w.tgt.as<int32_t>() : nullptr;  // (no targets in a prefill)
     if (packed) {

@@ -992,6 +992,29 @@ SeqPack seq_pack(const HostModel& hm, SeqShape sh, const std::vector<float>& lat
     return p;
 }
 
+// The kernel's time goes with its workgroups, whose eight tiles of 16 tokens cost the same however full they are; the
+// layered kernels' time goes with the rows, the sequences (attention) and their launches. So many sequences of a few tokens
+// are the layered body's: 65536 of one token, D128 H256, two blocks without attention, 1878 us in the kernel and 538
+// layered, of four tokens 1966 and 1437, of six 2023 and 2143; with attention and three blocks, of one token 4548 and 3516,
+// of two 4586 and 4165, of three 4622 and 4864. With 256 workgroups (2048 such sequences) the launches decide and the
+// kernel is the faster one at one token too (78 and 101, 171 and 301). From six tokens on it is always the faster one, also
+// where a workgroup is filled worst (131072 tokens of D128 H128 without attention: T = 8 582 and 881 us, T = 17 589 and
+// 901, T = 33 582 and 914, T = 65 580 and 917). The two estimates are nanoseconds on the whole chip without the head, fitted
+// to forwards and prefills of 20 models, T 1 to 128, 1 to 524288 sequences: the body they take was the faster one or within
+// 1 % of it in 99.6 % of 2805 measurements and never more than 9 % behind.
+bool seq_pays(SeqShape sh, int B, int T, int steps, int attns, int heads) {
+    if (T > 8) return true;
+    const int seqs = 8 / ((T + 15) / 16), slots = sh.dt == 1 && sh.nd == 0 ? 512 : 256;  // workgroups at once
+    const double wgs = (double)round_up((B + seqs - 1) / seqs, slots);
+    const double step = sh.dt == 2 ? (sh.ht == 2 ? 82 : sh.ht == 3 ? 94 : 111)
+                        : sh.nd    ? (sh.ht == 1 ? 33 : 42)
+                                   : (sh.ht == 1 ? 28 : 57);
+    const double kernel = wgs * (steps * step + attns * heads * 18.4);
+    const double row = 0.5 + steps * (sh.dt == 2 ? 1.4 + 0.2 * sh.ht : 1.05) + attns * (0.6 + 0.6 * sh.dt);
+    const double layered = 35000.0 * steps + 25000.0 * attns + B * (attns * heads * 3.1 + T * row);
+    return kernel <= layered;
+}
+
 bool seq_fits(const SeqArgs& a) { return a.shape.dt > 0 && a.T >= 1 && a.T <= kSeqMaxT && a.B >= 1; }
 
 hipError_t launch_seq(const SeqArgs& a, hipStream_t s) {

@@ -72,6 +72,8 @@ struct SeqArgs {
 };
 // Whether the kernel takes sequences of this length of a model whose shape it takes.
 bool seq_fits(const SeqArgs& a);
+// Whether it is the faster body there, for B sequences through `steps` rule steps and `attns` attention blocks in all.
+bool seq_pays(SeqShape sh, int B, int T, int steps, int attns, int heads);
 hipError_t launch_seq(const SeqArgs& a, hipStream_t s);
 
 }  // namespace mg

@@ -146,3 +146,47 @@ def test_many_steps():
             out[mode] = m.forward_batch(ids)["logits"], s.prefill(ids, lens)[0], s.step(ids[:, 0])[0]
         for a, b in zip(out["auto"], out["limbs"]):
             assert_close(a, b, rtol=2e-5, what=f"{blocks}")
+
+
+# D, H, heads, blocks, T, sequences, whether the one-kernel body is the faster one there: both sides of the line
+FILL = [
+    (128, 256, 0, [(1, 2, 1)] * 2, 1, 2048, True),
+    (128, 256, 0, [(1, 2, 1)] * 2, 1, 8192, False),
+    (128, 128, 0, [(1, 2, 1)] * 2, 4, 65536, False),
+    (128, 128, 0, [(1, 2, 1)] * 2, 6, 65536, True),
+    (32, 64, 0, [(2, 2, 1)], 1, 8192, True),
+    (32, 64, 0, [(2, 2, 1)], 1, 32768, False),
+    (96, 160, 4, [(1, 2, 1)] * 2, 1, 8192, True),
+    (96, 160, 4, [(1, 2, 1)] * 2, 1, 32768, False),
+    (96, 160, 4, [(1, 2, 1)] * 2, 3, 32768, True),
+]
+
+
+@pytest.mark.parametrize("D,H,heads,blocks,T,B,one", FILL)
+def test_short_sequences_take_the_faster_body(D, H, heads, blocks, T, B, one):
+    """Many sequences of a few tokens leave the kernel's tiles mostly empty and take the layered body (forward, prefill
+    and scoring with a short context), a few of them or longer ones the kernel; the same outputs either way."""
+    spec = tiny_spec(blocks, V=131, D=D, H=H, heads=heads, window=64 if heads else 0, context=128, tied=False)
+    data = uniform_model_bytes(spec, seed=8, scale=0.3)
+    m, om = Model(data), oracle_model(data)
+    ids = synth.token_ids(79, f"fill{D}{T}", (B, T), 131)
+    got, prof = _classes(m, lambda: m.forward_batch(ids)["logits"])
+    assert ("sequence_body" in prof) == one and ("gemm_glu" in prof) != one, prof
+    for b in (0, 1, 15, 16, B // 2, B - 1):
+        assert_close(got[b], om.forward_all(ids[b:b + 1])[0], what=f"sequence {b}")
+    if B <= 8192:
+        s = m.sessions(B, 128)
+        (lg, _, _), prof = _classes(m, lambda: s.prefill(ids))
+        assert ("sequence_body" in prof) == one, prof
+        assert_close(lg, got[:, -1], rtol=2e-5, what="prefill")
+        nexts = ids[::-1, 0].copy()
+        after = s.step(nexts)[0]
+        for b in (0, 17, B - 1):
+            assert_close(after[b], om.call(np.append(ids[b], nexts[b])), what=f"step of session {b}")
+    doc = ids.ravel()[:B + T - 1]  # about B windows of T tokens
+    (lp,), prof = _classes(m, lambda: score_sequences(m, [doc], T))
+    assert ("sequence_body" in prof) == one, prof
+    for t in (1, 2, len(doc) // 2, len(doc) - 1):
+        want = om.call(doc[max(0, t - T):t]).astype(np.float64)
+        want = want[doc[t]] - want.max() - np.log(np.exp(want - want.max()).sum())
+        assert abs(lp[t - 1] - want) <= 1e-4 * max(1.0, abs(want)), t
