@@ -1065,14 +1065,45 @@ bool seq_usable(mg_model* m, int B, int T) {
     return seq_fits(a) && seq_pays(a.shape, B, T, m->nbs, m->nattn, m->heads);
 }
 
-void run_seq(mg_model* m, const SeqArgs& a, hipStream_t s) {
-    double ops = 0;
-    if (m->prof.on) {
-        const double M = (double)a.B * a.T, D = m->D, H = m->H;
-        ops = 2.0 * M * (m->nbs * (D * D + 6 * D * H + 2 * D * H) + m->nattn * 4 * D * D);
+// Multiply-adds the kernel runs for a sequence of len positions of which the head reads `count` from `first` on: every block
+// but the last over all positions; of the last one the latch over all, and the products only in the 16-position tiles that
+// those rows, or with attention the keys they attend, lie in.
+double seq_macs(const mg_model* m, int len, int first, int count) {
+    const double D = m->D, rule = 8.0 * D * m->H;
+    const int span = m->window > 0 ? std::min(m->window, m->cap) : m->cap;
+    const int end = std::min(len, (first + count + 15) / 16 * 16);
+    const double out = end - first / 16 * 16, keys = end - std::max(first - span + 1, 0) / 16 * 16;
+    double macs = 0;
+    for (const DevBlock& b : m->blocks) {
+        const bool last = &b == &m->blocks.back();
+        macs += (double)len * b.steps * (D * D + rule);
+        if (last && b.steps > 0) macs -= (len - (b.attn ? keys : out)) * rule;
+        if (b.attn) macs += last ? (3 * keys + out) * D * D : 4.0 * len * D * D;
     }
-    // ids in, the final rows' limb planes and scales out
-    ProfScope ps(m->prof, K_SEQ, s, (double)a.B * a.T * (8.0 + 3.0 * m->Dp), ops);
+    return macs;
+}
+
+// rows, lens: the host's copies of a.rows and a.lens, where it has them.
+void run_seq(mg_model* m, const SeqArgs& a, hipStream_t s, const int4* rows = nullptr, const int32_t* lens = nullptr) {
+    double bytes = 0, ops = 0;
+    if (m->prof.on) {
+        std::vector<int32_t> copy;
+        if (a.lens && !lens) {
+            copy.resize(a.B);
+            HIPCHECK(hipMemcpyAsync(copy.data(), a.lens, (size_t)a.B * 4, hipMemcpyDeviceToHost, s));
+            HIPCHECK(hipStreamSynchronize(s));
+            lens = copy.data();
+        }
+        for (int b = 0; b < a.B; b++) {
+            const int len = lens ? std::min(lens[b], a.T) : a.T;
+            const int first = rows ? rows[b].x : a.last_only ? len - 1 : 0;
+            const int count = rows ? rows[b].y : a.last_only ? 1 : len;
+            ops += 2.0 * seq_macs(m, len, first, count);
+            // ids in, the limb planes and scales of the rows the head reads out
+            bytes += 4.0 * len + count * (4.0 + 3.0 * m->Dp);
+        }
+    }
+    ProfScope ps(m->prof, K_SEQ, s, bytes, ops);
     HIPCHECK(launch_seq(a, s));
 }
 
@@ -1626,7 +1657,7 @@ int mg_score_sequences(mg_model* m, const int32_t* tokens, const long long* offs
             if (seq) {
                 SeqArgs sq = seq_args(m, B, T, ids_d);
                 sq.rows = rows_d; sq.lens = len_d;
-                run_seq(m, sq, s);
+                run_seq(m, sq, s, h_rows.data(), h_len.data());
             } else {
                 BodyCtx c;
                 c.B = B; c.T = T; c.ids = ids_d;

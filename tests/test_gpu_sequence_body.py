@@ -190,3 +190,44 @@ def test_short_sequences_take_the_faster_body(D, H, heads, blocks, T, B, one):
         want = om.call(doc[max(0, t - T):t]).astype(np.float64)
         want = want[doc[t]] - want.max() - np.log(np.exp(want - want.max()).sum())
         assert abs(lp[t - 1] - want) <= 1e-4 * max(1.0, abs(want)), t
+
+
+@pytest.mark.parametrize("shape", [SHAPES[0], SHAPES[6], SHAPES[8], SHAPES[9], (128, 160, 4, 64, [(1, 2, 1)] * 2)])
+def test_profile_counts_what_runs(shape):
+    """The profiler's work of the kernel, wave by wave as it runs: a 16-token tile past a sequence's end does nothing, and
+    the last block's products run only where a row the head reads depends on them."""
+    D, H, heads, window, blocks = shape
+    m = Model(_build(shape))
+    Dp = -(-D // 64) * 64
+
+    def want(seqs):
+        ops = out = 0
+        for n, first, count in seqs:
+            for t in range(-(-n // 16)):
+                tokens = min(16, n - 16 * t)
+                read = 16 * t < first + count and 16 * t + 15 >= first
+                key = 16 * t < first + count and 16 * t + 15 >= first - window + 1
+                for i, (steps, _, _) in enumerate(blocks):
+                    last = i + 1 == len(blocks)
+                    for st in range(steps):
+                        ops += 2 * tokens * D * D
+                        if not last or st + 1 < steps or (key if heads else read):
+                            ops += 2 * tokens * 8 * D * H
+                    if heads:
+                        ops += 2 * tokens * D * D * (3 * (not last or key) + (not last or read))
+            out += 4 * n + count * (4 + 3 * Dp)
+        return out, ops
+
+    def check(fn, seqs):
+        prof = _classes(m, fn)[1]["sequence_body"]
+        assert prof[2:] == want(seqs), (shape, seqs[:3])
+
+    ids = synth.token_ids(80, "prof", (9, 128), 131)
+    check(lambda: m.forward_batch(ids), [(128, 0, 128)] * 9)
+    check(lambda: m.forward_batch(ids[:, :33].copy()), [(33, 0, 33)] * 9)
+    for n in (1, 16, 17, 45, 128):
+        check(lambda: m.call(ids[0, :n]), [(n, n - 1, 1)])
+    lens = np.array([1, 16, 17, 33, 64, 65, 80, 127, 128], np.int32)
+    check(lambda: m.sessions(9, 128).prefill(ids, lens), [(n, n - 1, 1) for n in lens.tolist()])
+    # a first window of the context's length, scored at all its targets, then one of that length per later target
+    check(lambda: score_sequences(m, [ids[0]], 40), [(40, 0, 40)] + [(40, 39, 1)] * 87)
