@@ -1403,6 +1403,7 @@ hipError_t launch_gemm_fa(int epi, const GemmArgs& a, hipStream_t stream) {
 
 hipError_t launch_gemm_c2(const GemmArgs& a, hipStream_t stream) {
     if (a.Kp <= 0 || a.M < 0 || a.nvalid <= 0 || (!a.out && !a.out_i32)) return hipErrorInvalidValue;
+    if (a.a_row != a.Kp || a.ldw != a.Kp) return hipErrorInvalidValue;  // Row16 takes rows without gaps
     if (a.M == 0) return hipSuccess;
     const long long tiles = (long long)((a.nvalid + GEMM_BN - 1) / GEMM_BN) * ((a.M + GEMM_BM - 1) / GEMM_BM);
     const long long thin = (long long)((a.nvalid + THIN - 1) / THIN) * ((a.M + THIN - 1) / THIN);
@@ -1412,7 +1413,7 @@ hipError_t launch_gemm_c2(const GemmArgs& a, hipStream_t stream) {
         return hipGetLastError();
     }
     const bool whole = a.Kp % GEMM_BK == 0 && a.nvalid % GEMM_BN == 0 && a.ldo % 4 == 0 && ((uintptr_t)a.out & 15) == 0 &&
-                       ((uintptr_t)a.A & 15) == 0 && ((uintptr_t)a.W & 15) == 0;
+                       ((uintptr_t)a.out_i32 & 15) == 0 && ((uintptr_t)a.A & 15) == 0 && ((uintptr_t)a.W & 15) == 0;
     if (whole) hipLaunchKernelGGL(gemm_c2_kernel<false>, dim3(xcd_grid((int)tiles)), dim3(256), 0, stream, a);
     else hipLaunchKernelGGL(gemm_c2_kernel<true>, dim3(xcd_grid((int)tiles)), dim3(256), 0, stream, a);
     return hipGetLastError();

@@ -49,13 +49,14 @@ constexpr int GEMM_BM = 64;
 constexpr int GEMM_BK = 64;
 
 struct GemmArgs {
-    // Limb-expanded A (fragment layout) with one scale per token row; or plain row-major int8 A (c2).
+    // Limb-expanded A (fragment layout) with one scale per token row; or plain row-major int8 A, [M][Kp] without gaps
+    // (c2: any K and address).
     const int8_t* A = nullptr;
-    long long a_row = 0;              // c2: row stride
+    long long a_row = 0;              // c2: Kp
     const float* As = nullptr;        // per-row limb scale
-    // W: fragment layout (limb-expanded path) or row-major [Np][ldw] (c2).
+    // W: fragment layout (limb-expanded path) or row-major [nvalid][Kp] without gaps (c2: any K, N and address).
     const int8_t* W = nullptr;
-    int ldw = 0;
+    int ldw = 0;                      // c2: Kp
     int M = 0, Np = 0, Kp = 0;
     int nvalid = 0;                   // output channels that exist (the rest are padding)
     float wscale = 1.0f;

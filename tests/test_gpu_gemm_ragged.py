@@ -40,3 +40,24 @@ def test_ragged_exact(M, K, N, shift):
             assert torch.equal(C.view(torch.int32), wantf.view(torch.int32))
         for t in (pad, cpad.view(torch.int32)):  # nothing around the outputs is written
             assert bool((t[:shift] == 7).all()) and bool((t[shift + M * N:] == 7).all())
+
+
+@pytest.mark.parametrize("M", [64 * 64, 64 * 64 + 9])
+@pytest.mark.parametrize("with_c", [False, True])
+def test_only_the_accumulators_unaligned(M, with_c):
+    """Whole tiles of aligned operands (64 of them, and a partial row of tiles) and the int32 output alone at an address of
+    no 16 bytes, which the whole-tile kernel's 16-byte stores do not take."""
+    K, N = 64, 128
+    rng = np.random.default_rng(M)
+    A, W = rng.integers(-128, 128, (M, K), np.int8), rng.integers(-128, 128, (N, K), np.int8)
+    s = (1e-3 + rng.random(N)).astype(np.float32)
+    dA, dW, ds = (torch.from_numpy(x).cuda() for x in (A, W, s))
+    want = (dA.double() @ dW.double().T).round().to(torch.int32)
+    pad = torch.full((M * N + 64,), 7, dtype=torch.int32, device="cuda")
+    acc = pad[1:1 + M * N].view(M, N)
+    C = torch.empty((M, N), device="cuda") if with_c else None
+    gemm_i8_device(dA, dW, ds, C, acc, torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(acc, want)
+    assert bool((pad[:1] == 7).all()) and bool((pad[1 + M * N:] == 7).all())
+    if with_c:
+        assert torch.equal(C.view(torch.int32), (want.float() * ds).view(torch.int32))
