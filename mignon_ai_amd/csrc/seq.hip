@@ -13,7 +13,7 @@
 // in that order once (seq_pack). A row's maxima and sums combine four lanes (two shuffles).
 //
 // Activations are expanded to three base-256 digits with one scale per row (scale = amax / 127, digits of
-// round(x * 127 * 65536 / amax): 0.5 / 8323072 of the row's maximum, the limb planes' own resolution).
+// round(x * 127 * 65536 / amax), off by at most 0.75 / 8323072 of the row's maximum and without a mean: digits23_4).
 //
 // Weights are read by the workgroup as a stream of units of UF fragments (1 KiB each) in the order of use (a block's rule
 // steps read the same units again, so that the stream is no longer than the weights whatever the step count), moved
@@ -134,31 +134,6 @@ __device__ __forceinline__ float abs_max(const float (&v)[N]) {
     return m;
 }
 
-struct Scale {
-    float s, inv;
-};
-__device__ __forceinline__ Scale digit_scale(float amax) {
-    if (amax < kTinyAmax) return Scale{0.0f, 0.0f};
-    return Scale{amax / 127.0f, 8323072.0f / amax};  // 127 * 65536
-}
-
-// The digit words of four values: q = round(x * inv) = 65536 q0 + 256 q1 + q2, |q| <= 127 * 65536. With
-// z = q + 0x8080, byte 2 of z is q0 and bytes 1 and 0 are q1 and q2 with bit 7 flipped. (x * inv + 0x8080 is rounded to
-// a multiple of a half or less by the fused multiply-add, then to the nearest integer by the conversion.)
-__device__ __forceinline__ uint32_t digit_z(float x, float inv) {
-    uint32_t z;
-    asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(z) : "v"(fmaf(x, inv, 32896.0f)));
-    return z;
-}
-__device__ __forceinline__ void digits4(float x0, float x1, float x2, float x3, float inv, int& w0, int& w1, int& w2) {
-    const uint32_t z0 = digit_z(x0, inv), z1 = digit_z(x1, inv), z2 = digit_z(x2, inv), z3 = digit_z(x3, inv);
-    const uint32_t a01 = __builtin_amdgcn_perm(z1, z0, 0x05010400u);
-    const uint32_t a23 = __builtin_amdgcn_perm(z3, z2, 0x05010400u);
-    w2 = (int)(__builtin_amdgcn_perm(a23, a01, 0x05040100u) ^ 0x80808080u);
-    w1 = (int)(__builtin_amdgcn_perm(a23, a01, 0x07060302u) ^ 0x80808080u);
-    w0 = (int)(__builtin_amdgcn_perm(z1, z0, 0x0c0c0602u) | __builtin_amdgcn_perm(z3, z2, 0x06020c0cu));
-}
-
 // Operand registers of NK K steps from a lane's 16 values per step (value 4j + r of step k: channel 64k + 16j + 4g + r).
 template <int NK, int N>
 __device__ __forceinline__ void expand(const float (&v)[N], float inv, v4i (*d)[3]) {
@@ -168,7 +143,7 @@ __device__ __forceinline__ void expand(const float (&v)[N], float inv, v4i (*d)[
         for (int j = 0; j < 4; j++) {
             int w0, w1, w2;
             const int i = 16 * k + 4 * j;
-            digits4(v[i], v[i + 1], v[i + 2], v[i + 3], inv, w0, w1, w2);
+            digits23_4(v[i], v[i + 1], v[i + 2], v[i + 3], inv, w0, w1, w2);
             d[k][0][j] = w0;
             d[k][1][j] = w1;
             d[k][2][j] = w2;
@@ -452,7 +427,7 @@ __global__ __launch_bounds__(512)
                 for (int ti = 0; ti < 4 * DT; ti++) stg((float4*)(d + 16 * ti), make_float4(n[4 * ti], n[4 * ti + 1], n[4 * ti + 2], n[4 * ti + 3]));
             }
             {
-                const Scale sc = digit_scale(nm);
+                const DigitScale sc = digit_scale(nm);
                 v4i nd[DT][3];
                 expand<DT>(n, sc.inv, nd);
                 const float sw = sc.s * B.ssel;
@@ -523,7 +498,7 @@ __global__ __launch_bounds__(512)
                 const bool hasl = t >= dl;
                 const int back = hasl ? dl : 0;
                 const float lm = hasl ? *(const float*)(smem + C::o_nmax + 4 * (lrow - back)) : 0.0f;
-                const Scale sc = digit_scale(fmaxf(fmaxf(nm, lm), row_max4(gm)));
+                const DigitScale sc = digit_scale(fmaxf(fmaxf(nm, lm), row_max4(gm)));
                 xsw = sc.s * B.s1;
                 expand<DT>(n, sc.inv, xd);
                 expand<DT>(sb, sc.inv, xd + 2 * DT);
@@ -580,7 +555,7 @@ __global__ __launch_bounds__(512)
             }
             // cur = (1 - g) cur + g o, in the same manner
             v4i hd[HT][3];
-            const Scale sc = digit_scale(row_max4(abs_max(h)));
+            const DigitScale sc = digit_scale(row_max4(abs_max(h)));
             const float hsw = sc.s * B.s2;
             expand<HT>(h, sc.inv, hd);
             constexpr int NU = 4 * DT / C::HW;
@@ -645,7 +620,7 @@ __global__ __launch_bounds__(512)
                     const float inv = rms_inv();
 #pragma unroll
                     for (int ti = 0; ti < 4 * DT; ti++) scale_by(inv, ti, ld4(v_off + V_AG + 64 * ti), n);
-                    const Scale sc = digit_scale(row_max4(abs_max(n)));
+                    const DigitScale sc = digit_scale(row_max4(abs_max(n)));
                     sw = sc.s * B.sqkv;
                     expand<DT>(n, sc.inv, nd);
                 }
@@ -774,7 +749,7 @@ __global__ __launch_bounds__(512)
                         const float4 x = ld4(x_off + 64 * ti);
                         att[4 * ti] = x.x; att[4 * ti + 1] = x.y; att[4 * ti + 2] = x.z; att[4 * ti + 3] = x.w;
                     }
-                    const Scale sc = digit_scale(row_max4(abs_max(att)));
+                    const DigitScale sc = digit_scale(row_max4(abs_max(att)));
                     osw = sc.s * B.so;
                     expand<DT>(att, sc.inv, nd);
                 }

@@ -6,9 +6,20 @@
 // (0 = success).
 #include <hip/hip_runtime.h>
 
+#include "common.hpp"
 #include "kernels.hpp"
 
 namespace {
+
+// The digits of four elements a thread, put together again.
+__global__ void digits23_kernel(const float* x, int n4, float amax, int32_t* q) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n4) return;
+    int w0, w1, w2;
+    mg::digits23_4(x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3], mg::digit_scale(amax).inv, w0, w1, w2);
+    for (int e = 0; e < 4; e++)
+        q[4 * i + e] = 65536 * (int8_t)(w0 >> 8 * e) + 256 * (int8_t)(w1 >> 8 * e) + (int8_t)(w2 >> 8 * e);
+}
 
 int finish(hipError_t launched) {
     if (launched != hipSuccess) return (int)launched;
@@ -106,6 +117,13 @@ int mgt_attention_step_packed(const int32_t* pos, const float* qkv, uint32_t* kp
 int mgt_export_kv_packed(int B, int T, int D, int heads, int cap, const int32_t* lens, const float* qkv,
                          uint32_t* kpack, uint32_t* vpack, float* kscale, float* vscale) {
     return finish(mg::launch_export_kv_packed(B, T, D, heads, cap, lens, qkv, kpack, vpack, kscale, vscale, nullptr));
+}
+
+// q of digits23_4 for 4 * n4 values of a row whose largest magnitude is amax.
+int mgt_digits23(const float* x, int n4, float amax, int32_t* q) {
+    if (n4 <= 0) return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL(digits23_kernel, dim3((n4 + 255) / 256), dim3(256), 0, nullptr, x, n4, amax, q);
+    return finish(hipGetLastError());
 }
 
 }  // extern "C"

@@ -78,6 +78,7 @@ def lib():
             "mgt_attention_step": [p, p, p, p, i, i, i, i, i, i, p, p, p, i],
             "mgt_attention_step_packed": [p, p, p, p, p, p, i, i, i, i, i, i, p, p, p, i],
             "mgt_export_kv_packed": [i, i, i, i, i, p, p, p, p, p, p],
+            "mgt_digits23": [p, i, ctypes.c_float, p],
         }
         for name, args in sig.items():
             fn = getattr(L, name)
