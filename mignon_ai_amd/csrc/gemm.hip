@@ -999,11 +999,13 @@ struct Row16 {
     }
 };
 
-// RAGGED: K no multiple of 64, N no multiple of 128 or an operand or C not 16-byte aligned: operands through Row16
-// (row-major [M][K] and [N][K] as the caller has them), C in rows of 16-byte or 4-byte stores. It replaces padded copies
-// of both operands and the wait for them (they died with the call): 100000 x 500 x 1000 224 -> 164 us, 100000 x 512 x
-// 1001 292 -> 166, 20000 x 100 x 777 93 -> 28, 2 x 1446 x 308 37 -> 8.5.
-template <bool RAGGED>
+// RAGGED: N no multiple of 128 or an operand or output not 16-byte aligned: C in rows of 16-byte or 4-byte stores, rows of W
+// past the last repeated. RAGGED_K: K no multiple of 64 or A or W not aligned: operands through Row16 (row-major [M][K] and
+// [N][K] as the caller has them). Together they replace padded copies of both operands and the wait for them (they died
+// with the call): 100000 x 500 x 1000 224 -> 164 us, 100000 x 512 x 1001 292 -> 166, 20000 x 100 x 777 93 -> 28, 2 x 1446 x
+// 308 37 -> 8.5. Where only N is ragged the loads go without Row16's checks: 100000 x 1536 x 1000 314 us with them, 299
+// without, 307 with a padded copy of W; 100000 x 384 x 1000 122, 114 and 122; 100000 x 1024 x 308 85, 79 and 92.
+template <bool RAGGED_K, bool RAGGED>
 __global__ __launch_bounds__(256) void gemm_c2_kernel(GemmArgs g) {
     __shared__ __align__(16) int8_t Ws[2][GEMM_BN * LDSR];
     __shared__ __align__(16) int8_t As[2][GEMM_BM * LDSR];
@@ -1027,7 +1029,7 @@ __global__ __launch_bounds__(256) void gemm_c2_kernel(GemmArgs g) {
     const Row16 w_row[2] = {Row16(g.W, n0 + (tid >> 2), g.nvalid, g.Kp), Row16(g.W, n0 + 64 + (tid >> 2), g.nvalid, g.Kp)};
     const Row16 a_rowp(g.A, a_m, g.M, g.Kp);
     auto gload = [&](int k0) {
-        if constexpr (RAGGED) {
+        if constexpr (RAGGED_K) {
 #pragma unroll
             for (int i = 0; i < 2; i++) {
                 const int c = tid + i * 256;
@@ -1038,7 +1040,8 @@ __global__ __launch_bounds__(256) void gemm_c2_kernel(GemmArgs g) {
 #pragma unroll
             for (int i = 0; i < 2; i++) {
                 int c = tid + i * 256;
-                wreg[i] = *(const v4i*)(g.W + (long long)(n0 + (c >> 2)) * g.ldw + k0 + (c & 3) * 16);
+                const int n = RAGGED ? min(n0 + (c >> 2), g.nvalid - 1) : n0 + (c >> 2);
+                wreg[i] = *(const v4i*)(g.W + (long long)n * g.ldw + k0 + (c & 3) * 16);
             }
             areg = a_ok ? *(const v4i*)(a_base + k0) : v4i{0, 0, 0, 0};
         }
@@ -1058,7 +1061,7 @@ __global__ __launch_bounds__(256) void gemm_c2_kernel(GemmArgs g) {
 #pragma unroll
         for (int tj = 0; tj < 2; tj++) acc[ti][tj] = v4i{0, 0, 0, 0};
 
-    const int ksteps = RAGGED ? (g.Kp + GEMM_BK - 1) / GEMM_BK : g.Kp / GEMM_BK;
+    const int ksteps = RAGGED_K ? (g.Kp + GEMM_BK - 1) / GEMM_BK : g.Kp / GEMM_BK;
     gload(0);
     sstore(0);
     __syncthreads();
@@ -1412,10 +1415,13 @@ hipError_t launch_gemm_c2(const GemmArgs& a, hipStream_t stream) {
         hipLaunchKernelGGL(gemm_thin_kernel, dim3((unsigned)thin), dim3(256), 0, stream, a);
         return hipGetLastError();
     }
-    const bool whole = a.Kp % GEMM_BK == 0 && a.nvalid % GEMM_BN == 0 && a.ldo % 4 == 0 && ((uintptr_t)a.out & 15) == 0 &&
-                       ((uintptr_t)a.out_i32 & 15) == 0 && ((uintptr_t)a.A & 15) == 0 && ((uintptr_t)a.W & 15) == 0;
-    if (whole) hipLaunchKernelGGL(gemm_c2_kernel<false>, dim3(xcd_grid((int)tiles)), dim3(256), 0, stream, a);
-    else hipLaunchKernelGGL(gemm_c2_kernel<true>, dim3(xcd_grid((int)tiles)), dim3(256), 0, stream, a);
+    auto aligned = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
+    const bool loads = a.Kp % GEMM_BK == 0 && aligned(a.A) && aligned(a.W);
+    const bool whole = loads && a.nvalid % GEMM_BN == 0 && a.ldo % 4 == 0 && aligned(a.out) && aligned(a.out_i32);
+    const dim3 grid(xcd_grid((int)tiles));
+    if (whole) hipLaunchKernelGGL((gemm_c2_kernel<false, false>), grid, dim3(256), 0, stream, a);
+    else if (loads) hipLaunchKernelGGL((gemm_c2_kernel<false, true>), grid, dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL((gemm_c2_kernel<true, true>), grid, dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 

@@ -61,3 +61,9 @@ def test_only_the_accumulators_unaligned(M, with_c):
     assert bool((pad[:1] == 7).all()) and bool((pad[1 + M * N:] == 7).all())
     if with_c:
         assert torch.equal(C.view(torch.int32), (want.float() * ds).view(torch.int32))
+
+
+@pytest.mark.parametrize("M,K,N", [(32705, 128, 127), (4096, 64, 1000), (4033, 192, 129), (70000, 64, 4), (8129, 384, 255)])
+def test_only_n_ragged(M, K, N):
+    """Whole, aligned K steps and channels that are not: rows of W past the last are repeated, not stored."""
+    test_ragged_exact(M, K, N, 0)
