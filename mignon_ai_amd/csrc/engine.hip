@@ -17,6 +17,7 @@
 #include <atomic>
 #include <cmath>
 #include <cstring>
+#include <exception>
 #include <limits>
 #include <memory>
 #include <mutex>
@@ -1148,6 +1149,13 @@ struct Staging {
     std::vector<std::unique_ptr<DevBuf>> bufs;
     Staging() = default;
     explicit Staging(mg_model* mm) : m(mm) {}
+    Staging(const Staging&) = delete;
+    Staging& operator=(const Staging&) = delete;
+    // A call that fails on the way still waits for the copies it began, from and to the caller's memory (the release of a
+    // call's own buffers waits by itself).
+    ~Staging() {
+        if (m && slot && std::uncaught_exceptions() > 0) (void)hipStreamSynchronize(m->stream);
+    }
     void* get(size_t bytes) {
         bytes = std::max<size_t>(bytes, 16);
         if (m && slot < kKeepSlots && bytes <= kKeepBytes) {
