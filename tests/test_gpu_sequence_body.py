@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 # D, H, heads, window, blocks: one entry per compiled variant, among them head widths of no whole groups of four or
-# below 16, several rule steps with dilations up to 32, a block without steps, windows of one key and of a whole tile
+# below 16, several rule steps with dilations up to 32, blocks without steps (the last one too), windows of one key, of a
+# whole tile and of the longest span
 SHAPES = [
     (32, 64, 0, 0, [(2, 2, 1)]),
     (64, 100, 0, 0, [(3, 3, 2), (1, 2, 1)]),
@@ -25,6 +26,8 @@ SHAPES = [
     (96, 128, 4, 64, [(1, 2, 1)] * 2),
     (100, 160, 4, 1, [(1, 2, 1)] * 2),
     (128, 256, 4, 17, [(2, 2, 1), (0, 2, 1), (1, 2, 2)]),
+    (24, 60, 2, 16, [(1, 2, 1), (0, 2, 1)]),
+    (128, 160, 4, 65, [(1, 2, 1), (2, 2, 1)]),
 ]
 
 
