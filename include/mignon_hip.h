@@ -97,7 +97,9 @@ int mg_model_sync(mg_model* m);
 void mg_model_free(mg_model* m);
 
 /* quant.Model.Call / Forward (internal/quant/model.go:120-137): next-token logits after the last
- * token, window truncated to max_context. logits: host double[V]. Returns V, or 0 for empty input. */
+ * token, window truncated to max_context. logits: host double[V]. Returns V, or 0 for empty input.
+ * The handle keeps pinned memory for max_context ids and V fp32 logits from the first call on. (Calls that take
+ * host pointers also keep their device buffers in the handle, at most eight of at most 16 MiB each.) */
 int mg_model_call(mg_model* m, const int32_t* ids, int n, double* logits);
 
 /* Teacher-forced batch: B sequences of T tokens, every position's next-token distribution at once.
@@ -294,7 +296,10 @@ int mg_gemm_i8(const int8_t* A, int M, int K, const int8_t* W, int N, const floa
 int mg_quantize_f32(const float* w, long long n, int8_t* q, float* scale, int flags, void* stream);
 
 /* Engine options, no reference counterpart: where two implementations of a stage exist, which one runs,
- * for every model of the process. Value 0 (the default) chooses automatically.
+ * for every model of the process. Value 0 (the default) chooses automatically. Small models (state size up
+ * to 128, hidden size up to 256, heads of up to 32 over spans of up to 65 keys) run sequences of up to 128 tokens
+ * through one kernel for the whole body; a value other than 0 of MG_OPT_GEMM_KERNEL, MG_OPT_ATTENTION_KERNEL,
+ * MG_OPT_SCAN_KERNEL or MG_OPT_OPERANDS selects among the layered kernels and takes those instead.
  *   MG_OPT_GEMM_KERNEL: MG_GEMM_STREAM streams weight tiles through LDS per token block;
  *     MG_GEMM_SLAB holds a weight slab in LDS and streams token tiles through it (used where the slab
  *     fits). Both give bit-identical results; automatic picks the slab kernel for large batches.

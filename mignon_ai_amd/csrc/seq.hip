@@ -20,18 +20,19 @@
 // straight from memory into four LDS slots: while unit u is used, units u + 1 to u + 3 are on their way, one barrier a
 // unit. A unit takes 1 to 2 thousand cycles and a load that misses the L2 about two thousand, so with only one unit
 // between a request and its use (through registers, two slots) every unit waited some 500 cycles: 1024 x 128 tokens of
-// the D128 model 756 -> 733 us, a call on 45 tokens 85.1 -> 81.8 us, scoring 60 documents 1486 -> 1432 us.
+// the D128 model 756 -> 733 us, a call on 45 tokens 85.1 -> 81.8 us, scoring 60 documents 1486 -> 1432 us (a slower card
+// than that of the comparison below).
 //
 // The latch recurrence g = lambda g + (1 - lambda) n runs over the tile's tokens as a scan over the 16 lanes of a DPP
 // row (pairs (a, b) composed in four steps), then over the tiles through LDS (each tile's composed pair).
 //
 // Bound by the matrix cores and the vector units together, which two waves per SIMD only partly overlap: per sequence
 // of 128 tokens of the D128 H256 two-block model about 95k matrix-core and 105k vector cycles per SIMD in 205k cycles.
-// Measured against the layered body, whole calls on one card: 1024 x 128 tokens of that model with logits and
-// log-probabilities 1277 -> 704 us (of which the head takes 300); 300 x 100 tokens of D96 H160 464 -> 281 us; 64 x 128
-// of D32 H64 123 -> 43 us; the next-token call on 45 tokens of D96 H160, its head over one row instead of 45, 253 ->
-// 85 us; scoring 60 documents with the D128 model, its last block only where a scored position depends on it, 3057 ->
-// 1515 us (all with the weights through registers).
+// Measured against the layered body, whole calls in turn on one card: 1024 x 128 tokens of that model with logits and
+// log-probabilities 1278 -> 709 us (about 200 of them the head's); 300 x 100 tokens of D96 H160 465 -> 277 us; 64 x 128
+// of D32 H64 123 -> 40.5 us; the next-token call on 45 tokens of D96 H160, its head over one row instead of 45, 245 ->
+// 82 us; scoring 60 documents with the D128 model, its last block only where a scored position depends on it, 3144 ->
+// 1423 us. Where it is not the faster body: seq_pays.
 #include <cmath>
 #include <cstring>
 #include <type_traits>
